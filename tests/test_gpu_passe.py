@@ -260,6 +260,33 @@ def test_attention_first_chunk_of_minus_inf_scores(k):
     assert np.abs(got - ref).max() <= 3e-6 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 72, 127, 128, 129, 1023, 1024, 1025, 1100])
+@pytest.mark.parametrize("tetes,kv,anneau,dec_v", [(64, 8, 0, 0), (6, 3, 0, 6), (4, 1, 5, 0), (8, 2, 70, 2)])
+def test_attention_chunk_edges(k, n, tetes, kv, anneau, dec_v):
+    """Position counts around the chunk sizes (8 up to 64 positions, then 64; 16 wavefronts a round),
+    heads that do not fill the XCDs, rings that wrap inside a chunk, values off 16-byte alignment, f16
+    and f32 caches. Bound: a score is a 64-term f32 dot of unit-variance values and a weight's relative
+    error is the score's absolute one (about 8 * 2^-24 * 64^0.5), averaged down over the positions:
+    1e-6 of max|out| as in the random cases above (they measure 2.4e-7)."""
+    print(f"attention n {n} heads {tetes}/{kv} ring {anneau}", flush=True)
+    rng = np.random.default_rng(n * 131 + tetes)
+    debut = 3 if not anneau else n // 2 + 3
+    cases = n + anneau if anneau else n + debut
+    p = ParamsAttention(tetes, kv, 64, debut, debut + n, cases if anneau else 0, 0.125, 0)
+    q = rng.standard_normal(tetes * 64).astype(np.float32)
+    ck = (rng.standard_normal(cases * kv * 64) * 0.5).astype(np.float16)
+    cv = rng.standard_normal(cases * kv * 64).astype(np.float16)
+    puits = rng.standard_normal(tetes).astype(np.float32)
+    ref64 = attention_f64(q, ck.view(np.uint16), cv.view(np.uint16), puits, p)
+    for appel, typ in ((k.attention, np.float16), (k.attention_kvf32, np.float32)):
+        dec = dec_v * (2 if typ == np.float32 else 1)
+        base = zeros(cv.size * np.dtype(typ).itemsize + dec)
+        base[dec:].copy_(torch.from_numpy(cv.astype(typ).view(np.uint8).copy()).to(base.device))
+        s = zeros(4 * 64 * tetes)
+        appel(vue(dev(q)), vue(dev(ck.astype(typ))), vue(base, dec), vue(dev(puits)), vue(s), p)
+        assert np.abs(hote(s, np.float32) - ref64).max() <= 1e-6 * np.abs(ref64).max(), typ
+
+
 def test_argmax_ties_nan_and_random(k):
     v = np.zeros(100_000, np.float32)
     v[0] = np.nan

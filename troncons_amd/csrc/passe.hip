@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "commun.hpp"
 #include "erreurs.hpp"
@@ -427,148 +428,235 @@ ecrire_kv(const float* __restrict__ k, const float* __restrict__ v, uint16_t* __
 // exp(sink - M)), M the largest of the scores and the sink. Query head h reads kv head
 // h / (heads / kv heads).
 //
-// One pass with a running softmax (Milakov & Gimelshein, "Online normalizer calculation for
-// softmax", 2018): the block's four wavefronts take chunks of 64 positions in turn (chunk c to
-// wavefront c mod 4). In a chunk, lane p scores position 64c + p; the wavefront's running maximum
-// moves to include the chunk's, and its running sum and its 64 running outputs (lane = dimension)
-// are rescaled by exp(old max - new max) before the chunk's terms are added; each position's weight
-// reaches the 64 dimensions through the wavefront's 64 LDS words. The four (max, sum, outputs) are
-// merged with the sink at the end, in wavefront order. No score array: any number of positions
-// fits in the block's 2 KiB of LDS. The caches hold f16 (attention) or f32 (attention_kvf32).
+// One block of 16 wavefronts per query head, one pass with a running softmax (Milakov & Gimelshein,
+// "Online normalizer calculation for softmax", 2018). A wavefront is eight groups of eight lanes;
+// a group takes one position at a time, lane j of it dimensions 8j .. 8j + 7 of its key and of its
+// value, so that a wavefront's load covers eight whole rows (a lane per row would touch 64 lines
+// for 16 bytes each). Chunks of 8 U positions go to the wavefronts in turn (chunk c to wavefront
+// c mod 16; position 8i + g of a chunk to group g). Each group keeps its own running maximum, sum
+// and outputs, rescaled by exp(old max - new max) once per chunk; lane i of a group takes the
+// exponential of its position 8i + g, the U weights reach its lanes through the wavefront's 64 LDS
+// words. Groups are merged by butterflies at the end, then the wavefronts and the sink in wavefront
+// order. No score array: any number of positions.
+//
+// What bounds it: a block reads its head's keys and values through one CU's vector memory path (2 MB
+// at 8192 positions) and spends about 250 VALU instructions per 64 positions on them; the blocks of a
+// kv head sit on one XCD, whose L2 then holds that head's rows for all of them. 64 heads over 8 kv
+// heads in f16: 274 -> 24 us at 8192 positions (one lane per position and four wavefronts before),
+// 9.2 -> 4.0 us at 128. The caches hold f16 (attention) or f32 (attention_kvf32).
 namespace trc {
-__device__ __forceinline__ float lire_kv(uint16_t b) { return f16_vers_f32(b); }
-__device__ __forceinline__ float lire_kv(float v) { return v; }
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+constexpr uint32_t FILS_ATTENTION = 1024;
+constexpr uint32_t VAGUES_ATTENTION = FILS_ATTENTION / 64u;
+constexpr uint32_t ATTENTION_COURTE = 64;  // positions up to which chunks hold 8 of them
 
-// q . k for one stored key row of 64 values, q in LDS as 16 float4: four interleaved partial
-// chains (dimensions 4u + 0..3 of each group of 16) added pairwise at the end.
-__device__ __forceinline__ float produit_cle(const f32x4* qs, const uint16_t* kr) {
-    const gptr<u32x4> k4 = glob<u32x4>(kr);
-    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (uint32_t b = 0; b < 8; ++b) {
-        const u32x4 w = k4[b];
-        const f32x4 qa = qs[2 * b], qb = qs[2 * b + 1];
-        a[0] = fmaf(qa.x, f16_vers_f32(w.x & 0xFFFFu), a[0]);
-        a[1] = fmaf(qa.y, f16_vers_f32(w.x >> 16), a[1]);
-        a[2] = fmaf(qa.z, f16_vers_f32(w.y & 0xFFFFu), a[2]);
-        a[3] = fmaf(qa.w, f16_vers_f32(w.y >> 16), a[3]);
-        a[0] = fmaf(qb.x, f16_vers_f32(w.z & 0xFFFFu), a[0]);
-        a[1] = fmaf(qb.y, f16_vers_f32(w.z >> 16), a[1]);
-        a[2] = fmaf(qb.z, f16_vers_f32(w.w & 0xFFFFu), a[2]);
-        a[3] = fmaf(qb.w, f16_vers_f32(w.w >> 16), a[3]);
-    }
-    return (a[0] + a[1]) + (a[2] + a[3]);
-}
-__device__ __forceinline__ float produit_cle(const f32x4* qs, const float* kr) {
-    const gptr<f32x4> k4 = glob<f32x4>(kr);
-    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (uint32_t b = 0; b < 16; ++b) {
-        const f32x4 w = k4[b], qv = qs[b];
-        a[0] = fmaf(qv.x, w.x, a[0]);
-        a[1] = fmaf(qv.y, w.y, a[1]);
-        a[2] = fmaf(qv.z, w.z, a[2]);
-        a[3] = fmaf(qv.w, w.w, a[3]);
-    }
-    return (a[0] + a[1]) + (a[2] + a[3]);
-}
-
-__device__ __forceinline__ float max_vague(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
-    return v;
-}
-__device__ __forceinline__ float somme_vague(float v) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
-    return v;
-}
-
+// Dimensions 8j .. 8j + 7 of a stored row. LARGE: the row is 16-byte aligned.
 template <typename T>
+using f16ou32 = std::conditional_t<sizeof(T) == 2, f16x8, f32x8>;
+template <bool LARGE>
+__device__ __forceinline__ f16x8 lire_brut(const uint16_t* p) {
+    if (LARGE) return *glob<f16x8>(p);
+    f16x8 h;
+#pragma unroll
+    for (uint32_t d = 0; d < 8; ++d) h[d] = __builtin_bit_cast(_Float16, uint16_t(glob<uint16_t>(p)[d]));
+    return h;
+}
+template <bool LARGE>
+__device__ __forceinline__ f32x8 lire_brut(const float* p) {
+    f32x8 r;
+    if (LARGE) {
+        const f32x4 a = glob<f32x4>(p)[0], b = glob<f32x4>(p)[1];
+        r = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+#pragma unroll
+        for (uint32_t d = 0; d < 8; ++d) r[d] = glob<float>(p)[d];
+    }
+    return r;
+}
+
+// v of the lane at xor 1, at xor 2, mirrored within its eight lanes (quad_perm, row_half_mirror).
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_MIROIR8 = 0x141;
+template <int DPP>
+__device__ __forceinline__ float voisin(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP, 0xF, 0xF, false));
+}
+// Sum and maximum over the eight lanes of a group; every lane gets the same bits.
+__device__ __forceinline__ float somme_groupe(float v) {
+    v += voisin<DPP_XOR1>(v);
+    v += voisin<DPP_XOR2>(v);
+    return v + voisin<DPP_MIROIR8>(v);
+}
+__device__ __forceinline__ float max_groupe(float v) {
+    v = fmaxf(v, voisin<DPP_XOR1>(v));
+    v = fmaxf(v, voisin<DPP_XOR2>(v));
+    return fmaxf(v, voisin<DPP_MIROIR8>(v));
+}
+// Lane j's share of the U = 8 sums over a group: sum over its lanes of s[j]. Each level hands the
+// half of the values that the partner keeps: 4 + 2 + 1 additions instead of 3 for each value.
+__device__ __forceinline__ float somme_transposee(const float (&s)[8], uint32_t j) {
+    float a[4], b[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const float garde = j < 4u ? s[i] : s[4 + i], donne = j < 4u ? s[4 + i] : s[i];
+        a[i] = garde + voisin<DPP_MIROIR8>(donne);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        const float garde = (j & 2u) == 0u ? a[i] : a[2 + i], donne = (j & 2u) == 0u ? a[2 + i] : a[i];
+        b[i] = garde + voisin<DPP_XOR2>(donne);
+    }
+    const float garde = (j & 1u) == 0u ? b[0] : b[1], donne = (j & 1u) == 0u ? b[1] : b[0];
+    return garde + voisin<DPP_XOR1>(donne);
+}
+__device__ __forceinline__ float somme_transposee(const float (&s)[1], uint32_t) { return somme_groupe(s[0]); }
+
+template <typename T, uint32_t U, bool LARGE>
 __device__ __forceinline__ void attention_tete(const float* __restrict__ q, const T* __restrict__ cache_k,
                                                const T* __restrict__ cache_v, const float* __restrict__ puits,
                                                float* __restrict__ sortie, const trc_params_attention& p) {
-    constexpr uint32_t VAGUES = FILS_PASSE / 64u;
-    __shared__ f32x4 qs[ATTENTION_DIM / 4];
-    __shared__ float poids[VAGUES][64];
-    __shared__ float sorties[VAGUES][ATTENTION_DIM];
-    __shared__ float maxima[VAGUES], sommes[VAGUES];
-    const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63u;
-    const uint32_t h = blockIdx.x;
-    const uint32_t hk = h / (p.tetes / p.tetes_kv);
+    static_assert(U == 1 || U == 8, "somme_transposee");
+    constexpr uint32_t RANGEES = 8u * U;  // positions per chunk
+    // rows of a lane in flight: f16 a whole chunk's keys and values, f32 (twice the registers) half of
+    // the keys, then half of the values
+    constexpr uint32_t LOT = sizeof(T) == 2 || U < 4u ? U : U / 2u;
+    __shared__ float poids[VAGUES_ATTENTION][64];
+    __shared__ float sorties[VAGUES_ATTENTION][ATTENTION_DIM];
+    __shared__ float maxima[VAGUES_ATTENTION], sommes[VAGUES_ATTENTION];
+    const uint32_t t = threadIdx.x, w = uint32_t(__builtin_amdgcn_readfirstlane(int(t >> 6)));
+    const uint32_t lane = t & 63u, g = lane >> 3, j = lane & 7u;
+    // blocks go round the XCDs in turn: the query heads of one kv head to the same one (8 kv heads)
+    const uint32_t hk = blockIdx.x % p.tetes_kv, h = hk * (p.tetes / p.tetes_kv) + blockIdx.x / p.tetes_kv;
     const uint64_t dkv = uint64_t(p.tetes_kv) * ATTENTION_DIM;
     const uint32_t n = p.fin - p.debut;
-    if (t < ATTENTION_DIM / 4u) qs[t] = glob<f32x4>(q + uint64_t(h) * ATTENTION_DIM)[t];
-    __syncthreads();
-
-    const T* cles = cache_k + uint64_t(hk) * ATTENTION_DIM;
-    const T* valeurs = cache_v + uint64_t(hk) * ATTENTION_DIM + lane;
-    float m = -INFINITY, z = 0.0f, o = 0.0f;
-    for (uint32_t c0 = 64u * w; c0 < n; c0 += 64u * VAGUES) {
-        const uint32_t pos0 = p.debut + c0;
-        const uint32_t case0 = p.anneau ? pos0 % p.anneau : pos0;  // slots of the chunk: case0 + k, wrapped
-        auto case_de = [&](uint32_t k) {
-            const uint32_t c = case0 + k;
-            return p.anneau && c >= p.anneau ? c - p.anneau : c;
-        };
-        const bool ok = c0 + lane < n;
-        const float s = ok ? produit_cle(qs, cles + uint64_t(case_de(lane)) * dkv) * p.echelle : -INFINITY;
-        const float m2 = fmaxf(m, max_vague(s));
-        // While every score so far is -inf (keys with an infinite component), m2 is -inf and
-        // exp(-inf - -inf) would be NaN: no term has weight yet, as in the reference, whose maximum
-        // includes the sink before any exponential (passe.cuh:306-371).
-        const float alpha = m == -INFINITY ? 0.0f : expf(m - m2);  // 0 for the first chunk (m = -inf)
-        const float e = m2 == -INFINITY ? 0.0f : expf(s - m2);      // 0 for lanes past the end
-        z = fmaf(z, alpha, somme_vague(e));
-        poids[w][lane] = e;  // read back by this wavefront only, in program order
-        const uint32_t nc = min(64u, n - c0);
-        float acc = 0.0f;
-        constexpr uint32_t LOT = 8;
-        for (uint32_t k0 = 0; k0 < nc; k0 += LOT) {
-            T vv[LOT];
+    const uint32_t case0 = p.anneau ? p.debut % p.anneau : p.debut;
+    const T* cles = cache_k + uint64_t(hk) * ATTENTION_DIM + 8u * j;
+    const T* valeurs = cache_v + uint64_t(hk) * ATTENTION_DIM + 8u * j;
+    float m = -INFINITY, z = 0.0f;  // m: the group's; z: the lane's share of the group's sum
+    f32x8 o = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    const float puits_h = puits[h];
+    if (RANGEES * w < n) {
+        const f32x8 qv = lire_brut<true>(q + uint64_t(h) * ATTENTION_DIM + 8u * j);
+        for (uint32_t c0 = RANGEES * w; c0 < n; c0 += RANGEES * VAGUES_ATTENTION) {
+            const uint32_t c = case0 + c0, tour = p.anneau && c >= p.anneau ? p.anneau : 0u;  // wave-uniform
+            const bool regulier = c0 + RANGEES <= n && (p.anneau == 0u || c - tour + RANGEES <= p.anneau);
+            // the rows of positions c0 + 8i + g, i = i0 .. i0 + LOT - 1 (past the end: the last one's)
+            auto lire_rangees = [&](const T* base, auto large, uint32_t i0, f16ou32<T>(&v)[LOT]) {
+                if (regulier) {
+                    const T* b0 = base + uint64_t(c - tour + g) * dkv;
 #pragma unroll
-            for (uint32_t u = 0; u < LOT; ++u) vv[u] = valeurs[uint64_t(case_de(min(k0 + u, nc - 1u))) * dkv];
+                    for (uint32_t i = 0; i < LOT; ++i)
+                        v[i] = lire_brut<decltype(large)::value>(b0 + 8u * (i0 + i) * dkv);
+                } else {
 #pragma unroll
-            for (uint32_t u = 0; u < LOT; ++u)
-                if (k0 + u < nc) acc = fmaf(poids[w][k0 + u], lire_kv(vv[u]), acc);
+                    for (uint32_t i = 0; i < LOT; ++i) {
+                        const uint32_t ci = case0 + min(c0 + 8u * (i0 + i) + g, n - 1u);
+                        v[i] = lire_brut<decltype(large)::value>(
+                            base + uint64_t(p.anneau && ci >= p.anneau ? ci - p.anneau : ci) * dkv);
+                    }
+                }
+            };
+            f16ou32<T> kv[LOT], vv[LOT];
+            lire_rangees(cles, std::true_type{}, 0u, kv);
+            if (LOT == U) lire_rangees(valeurs, std::bool_constant<LARGE>{}, 0u, vv);
+            float s[U];
+#pragma unroll
+            for (uint32_t i0 = 0; i0 < U; i0 += LOT) {
+                if (i0 > 0u) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    lire_rangees(cles, std::true_type{}, i0, kv);
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < LOT; ++i) {
+                    float a = qv[0] * float(kv[i][0]);
+#pragma unroll
+                    for (uint32_t d = 1; d < 8; ++d) a = fmaf(qv[d], float(kv[i][d]), a);
+                    s[i0 + i] = a;
+                }
+            }
+            if (LOT < U) {
+                __builtin_amdgcn_sched_barrier(0);
+                lire_rangees(valeurs, std::bool_constant<LARGE>{}, 0u, vv);
+            }
+            // lane j < U: the score of position c0 + 8j + g
+            const float som = somme_transposee(s, j) * p.echelle;
+            const float s_j = c0 + (U == 1u ? 0u : 8u * j) + g < n ? som : -INFINITY;
+            const float m2 = fmaxf(m, max_groupe(s_j));
+            // While every score so far is -inf (keys with an infinite component), m2 is -inf and
+            // exp(-inf - -inf) would be NaN: no term has weight yet, as in the reference, whose maximum
+            // includes the sink before any exponential (passe.cuh:306-371).
+            const float alpha = m == -INFINITY ? 0.0f : expf(m - m2);  // 0 for the first chunk (m = -inf)
+            const float e = m2 == -INFINITY || j >= U ? 0.0f : expf(s_j - m2);
+            z = fmaf(z, alpha, e);
+            m = m2;
+            poids[w][lane] = e;  // read back by this group only, in program order
+#pragma unroll
+            for (uint32_t d = 0; d < 8; ++d) o[d] *= alpha;
+#pragma unroll
+            for (uint32_t i0 = 0; i0 < U; i0 += LOT) {
+                if (i0 > 0u) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    lire_rangees(valeurs, std::bool_constant<LARGE>{}, i0, vv);
+                }
+                if (!regulier) {  // no value of a row past the end is used
+#pragma unroll
+                    for (uint32_t i = 0; i < LOT; ++i)
+                        if (c0 + 8u * (i0 + i) + g >= n) vv[i] = {};
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < LOT; ++i) {
+                    const float pi = poids[w][8u * g + i0 + i];
+#pragma unroll
+                    for (uint32_t d = 0; d < 8; ++d) o[d] = fmaf(pi, float(vv[i][d]), o[d]);
+                }
+            }
         }
-        o = fmaf(o, alpha, acc);
-        m = m2;
+    }
+    // the wavefront's eight groups: their common maximum, then the rescaled sums
+    float mv = m;
+#pragma unroll
+    for (int x = 8; x < 64; x <<= 1) mv = fmaxf(mv, __shfl_xor(mv, x));
+    const float f = m == -INFINITY ? 0.0f : expf(m - mv);
+    z = somme_groupe(z * f);
+#pragma unroll
+    for (int x = 8; x < 64; x <<= 1) z += __shfl_xor(z, x);
+#pragma unroll
+    for (uint32_t d = 0; d < 8; ++d) {
+        o[d] *= f;
+#pragma unroll
+        for (int x = 8; x < 64; x <<= 1) o[d] += __shfl_xor(o[d], x);
     }
     if (lane == 0) {
-        maxima[w] = m;
+        maxima[w] = mv;
         sommes[w] = z;
     }
-    sorties[w][lane] = o;
+    if (g == 0) {
+#pragma unroll
+        for (uint32_t d = 0; d < 8; ++d) sorties[w][8u * j + d] = o[d];
+    }
     __syncthreads();
     if (t < ATTENTION_DIM) {
-        const float puits_h = puits[h];
         float mg = puits_h;
 #pragma unroll
-        for (uint32_t v = 0; v < VAGUES; ++v) mg = fmaxf(mg, maxima[v]);
+        for (uint32_t v = 0; v < VAGUES_ATTENTION; ++v) mg = fmaxf(mg, maxima[v]);
         float zg = expf(puits_h - mg), og = 0.0f;
 #pragma unroll
-        for (uint32_t v = 0; v < VAGUES; ++v) {
-            const float f = expf(maxima[v] - mg);
-            zg = fmaf(sommes[v], f, zg);
-            og = fmaf(sorties[v][t], f, og);
+        for (uint32_t v = 0; v < VAGUES_ATTENTION; ++v) {
+            const float fv = expf(maxima[v] - mg);
+            zg = fmaf(sommes[v], fv, zg);
+            og = fmaf(sorties[v][t], fv, og);
         }
         sortie[uint64_t(h) * ATTENTION_DIM + t] = og / zg;
     }
 }
-}  // namespace trc
 
-extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
-attention(const float* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
+template <typename T, uint32_t U, bool LARGE>
+__global__ void __launch_bounds__(FILS_ATTENTION)
+attention(const float* __restrict__ q, const T* __restrict__ cache_k, const T* __restrict__ cache_v,
           const float* __restrict__ puits, float* __restrict__ sortie, trc_params_attention p) {
-    trc::attention_tete(q, cache_k, cache_v, puits, sortie, p);
+    attention_tete<T, U, LARGE>(q, cache_k, cache_v, puits, sortie, p);
 }
-
-extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
-attention_kvf32(const float* __restrict__ q, const float* __restrict__ cache_k, const float* __restrict__ cache_v,
-                const float* __restrict__ puits, float* __restrict__ sortie, trc_params_attention p) {
-    trc::attention_tete(q, cache_k, cache_v, puits, sortie, p);
-}
+}  // namespace trc
 
 // k and v copied unrounded into slot case_kv of f32 caches (passe.cuh:379-387).
 extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
@@ -750,25 +838,39 @@ int verifier_attention(trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puit
 }
 }  // namespace
 
+namespace {
+// One block per query head; chunks of 64 positions, or of 8 up to ATTENTION_COURTE positions, where
+// one 64-position chunk would leave 15 wavefronts idle (measured, us with chunks of 64 / of 8: 4.2 /
+// 4.0 at 64 positions, 4.0 / 4.5 at 128, 4.0 / 4.9 at 256, 4.4 / 6.1 at 512). Values that are not
+// 16-byte aligned (the contract asks it of the keys only) are read one by one.
+template <typename T>
+int lancer_attention(const char* nom, trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puits, trc_vue sortie,
+                     const trc_params_attention* p, void* flux) {
+    const int r = verifier_attention(q, cache_k, cache_v, puits, sortie, p, sizeof(T));
+    if (r != TRC_OK) return r;
+    auto lancer = [&](auto noyau) {
+        hipLaunchKernelGGL(noyau, dim3(p->tetes), dim3(trc::FILS_ATTENTION), 0, flux_de(flux),
+                           reinterpret_cast<const float*>(q.adresse), reinterpret_cast<const T*>(cache_k.adresse),
+                           reinterpret_cast<const T*>(cache_v.adresse), reinterpret_cast<const float*>(puits.adresse),
+                           reinterpret_cast<float*>(sortie.adresse), *p);
+    };
+    const bool long_ = p->fin - p->debut > trc::ATTENTION_COURTE, large = cache_v.adresse % 16 == 0;
+    if (large)
+        long_ ? lancer(trc::attention<T, 8, true>) : lancer(trc::attention<T, 1, true>);
+    else
+        long_ ? lancer(trc::attention<T, 8, false>) : lancer(trc::attention<T, 1, false>);
+    return trc::apres_lancement(nom);
+}
+}  // namespace
+
 extern "C" int trc_attention(trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puits, trc_vue sortie,
                              const trc_params_attention* p, void* flux) {
-    const int r = verifier_attention(q, cache_k, cache_v, puits, sortie, p, 2);
-    if (r != TRC_OK) return r;
-    hipLaunchKernelGGL(attention, dim3(p->tetes), dim3(trc::FILS_PASSE), 0, flux_de(flux),
-                       reinterpret_cast<const float*>(q.adresse), reinterpret_cast<const uint16_t*>(cache_k.adresse),
-                       reinterpret_cast<const uint16_t*>(cache_v.adresse), reinterpret_cast<const float*>(puits.adresse),
-                       reinterpret_cast<float*>(sortie.adresse), *p);
-    return trc::apres_lancement("attention");
+    return lancer_attention<uint16_t>("attention", q, cache_k, cache_v, puits, sortie, p, flux);
 }
 
 extern "C" int trc_attention_kvf32(trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puits, trc_vue sortie,
                                    const trc_params_attention* p, void* flux) {
-    const int r = verifier_attention(q, cache_k, cache_v, puits, sortie, p, 4);
-    if (r != TRC_OK) return r;
-    hipLaunchKernelGGL(attention_kvf32, dim3(p->tetes), dim3(trc::FILS_PASSE), 0, flux_de(flux), reinterpret_cast<const float*>(q.adresse),
-                       reinterpret_cast<const float*>(cache_k.adresse), reinterpret_cast<const float*>(cache_v.adresse),
-                       reinterpret_cast<const float*>(puits.adresse), reinterpret_cast<float*>(sortie.adresse), *p);
-    return trc::apres_lancement("attention_kvf32");
+    return lancer_attention<float>("attention_kvf32", q, cache_k, cache_v, puits, sortie, p, flux);
 }
 
 extern "C" int trc_ecrire_kv_f32(trc_vue k, trc_vue v, trc_vue cache_k, trc_vue cache_v, uint32_t dkv,
