@@ -356,3 +356,27 @@ def test_biased_router_equals_oracle_and_plain_router_without_bias():
     mots = boite.numpy()[:9].view(np.uint32)
     assert mots[0] == 91 and list(mots[1:5]) == [1, 2, 4, 3]
     assert (mots[5:9] == hote(pv, np.uint32)[:4]).all()
+
+
+@pytest.mark.parametrize("N", [63, 64, 65, 100, 256, 1000])
+@pytest.mark.parametrize("dims", [([96, 96, 2880], [2880, 2880, 96]), ([300, 300, 544], [544, 544, 320])])
+@pytest.mark.parametrize("entropie", ["moyenne", "forte"])
+def test_decoder_long_delta_tiles(k, N, dims, entropie):
+    """DELTA tiles around the length from which they are decoded as chains (64 macro-steps), whole and cut
+    short by the stream's end, rows of 3 to 90 blocks; `forte`: scales over all 256 exponents, whose
+    words are used faster than the 64 a macro-step that the chain translates ahead. Bytes equal the
+    oracle's."""
+    print(f"long DELTA tiles N {N} dims {dims} {entropie}", flush=True)
+    d = DimsExpert.de(*dims)
+    rng = np.random.default_rng(N)
+    blocs, biais = codeur.synth_expert(77, 0, N, d)
+    if entropie == "forte":
+        for b in blocs:
+            b.reshape(-1, 17)[:, 0] = rng.integers(0, 256, b.size // 17)
+    freqs = [codeur.tables([blocs[j]], d.lignes[j], d.colonnes[j] // 32) for j in range(3)]
+    partie, _ = codeur.partie(blocs, biais, freqs, d, N_delta=N, N_codes=16)
+    luts = O.luts_couche([[freqs[j][t] for t in range(4)] for j in range(3)])
+    empl, ctl = _decoder(k, partie, luts, dims=d)
+    assert list(ctl) == [0, 0, 0, 0]
+    oracle, octl = O.decoder_expert(partie, luts, d.lignes, d.colonnes)
+    assert list(octl) == [0, 0, 0, 0] and (oracle == empl).all()

@@ -32,8 +32,11 @@ constexpr int CTL_FORMAT = 1;
 constexpr int CTL_POINTEUR = 2;
 
 // Threads per block of the reference-API kernels (abi.rs:56-61 keeps these a launch detail).
-constexpr uint32_t FILS_ECHELLES = 128;  // 2 wavefronts = 4 DELTA tiles
+constexpr uint32_t FILS_ECHELLES = 256;  // 4 wavefronts: 4 long DELTA tiles, or 8 short ones
 constexpr uint32_t FILS_CODES = 256;     // 4 wavefronts = 8 CODES_CTX tiles
+// Tiles per block that the decoders' grids count on (kernels take any grid).
+constexpr uint32_t TUILES_BLOC_ECHELLES = 4;
+constexpr uint32_t TUILES_BLOC_CODES = 8;
 constexpr uint32_t FILS_BRUT = 256;
 constexpr uint32_t GEMV_FILS = 256;
 constexpr uint32_t GEMV_LIGNES_PAR_BLOC = 16;  // 8 half-wavefronts x 2 rows

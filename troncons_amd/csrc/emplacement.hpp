@@ -6,6 +6,7 @@
 #pragma once
 
 #include "anneau.hpp"
+#include "chaines.hpp"
 #include "commun.hpp"
 #include "entiers.hpp"
 #include "fusion_corps.hpp"
@@ -70,7 +71,9 @@ __device__ __forceinline__ uint32_t octets_hauts(uint32_t e0, uint32_t e1, uint3
 template <uint32_t FILS>
 struct LdsEchelles {
     uint2 lut[M];
-    __attribute__((aligned(OCTETS_ANNEAU))) uint8_t anneaux[(FILS / 32u) * OCTETS_ANNEAU];
+    // a ring per half-wavefront, or a chain zone per wavefront
+    __attribute__((aligned(OCTETS_ANNEAU))) uint8_t
+        anneaux[(FILS / 64u) * (CHAINE_OCTETS > 2u * OCTETS_ANNEAU ? CHAINE_OCTETS : 2u * OCTETS_ANNEAU)];
     __attribute__((aligned(16))) uint8_t med[MED_LDS_MAX];
 };
 
@@ -93,6 +96,15 @@ __device__ __forceinline__ void echelles_vers_emplacement(const DescFlux& fd, co
         med = s.med;
     }
     __syncthreads();
+    uint8_t* ech = mat + disp.echelles;
+    if (h.N >= CHAINE_N_MIN) {  // uniform
+        uint8_t* zone = s.anneaux + (threadIdx.x >> 6) * CHAINE_OCTETS;
+        if (R <= MED_LDS_MAX)
+            chaine_echelles<true>(fd, h, R, B, ech, s.lut, zone, s.med, fm.p, FILS / 64u, controle);
+        else
+            chaine_echelles<false>(fd, h, R, B, ech, s.lut, zone, s.med, fm.p, FILS / 64u, controle);
+        return;
+    }
 
     const Demi d = demi_courante();
     const Diviseur parB = Diviseur::de(B);
@@ -100,7 +112,6 @@ __device__ __forceinline__ void echelles_vers_emplacement(const DescFlux& fd, co
     const uint32_t nmacro = h.P / 128u;
     const uint32_t a_lut = adresse_lds(&s.lut[0]);
     const uint32_t a_anneau = adresse_lds(s.anneaux) + d.demi * OCTETS_ANNEAU;
-    uint8_t* ech = mat + disp.echelles;
     uint32_t hors_l = 0, pointeur = 0;
     for (uint32_t t0 = 2u * vague; t0 < h.T; t0 += 2u * n_vagues) {
         const uint32_t t = t0 + (d.haut ? 1u : 0u);

@@ -64,7 +64,7 @@ extern "C" void trc_grilles_decodeur(const trc_dims_expert* dims, uint32_t g1[3]
         td = td > tuiles(blocs) ? td : tuiles(blocs);
         tc = tc > tuiles(16 * blocs) ? tc : tuiles(16 * blocs);
     }
-    const uint32_t pe = trc::FILS_ECHELLES / 32, pc = trc::FILS_CODES / 32;
+    const uint32_t pe = trc::TUILES_BLOC_ECHELLES, pc = trc::TUILES_BLOC_CODES;
     g1[0] = au_moins_1((td + pe - 1) / pe);
     g1[1] = 3;
     g1[2] = 1;
@@ -115,7 +115,7 @@ extern "C" int trc_grilles_depuis_partie(const uint8_t* partie, size_t octets, u
     }
     for (int j = 0; j < 3; ++j)
         if (!vus[j][0] || !vus[j][1]) return usage("DELTA ou CODES_CTX absent pour une matrice");
-    const uint32_t pe = trc::FILS_ECHELLES / 32, pc = trc::FILS_CODES / 32;
+    const uint32_t pe = trc::TUILES_BLOC_ECHELLES, pc = trc::TUILES_BLOC_CODES;
     g1[0] = au_moins_1((td + pe - 1) / pe);
     g1[1] = 3;
     g1[2] = 1;
