@@ -851,7 +851,8 @@ __device__ __forceinline__ void corps_gemv_rapide(const Tache& tc, const PrepGem
             const uint32_t ax = (ent & ENT_X) | a_x;
             const f32x4 xa = lire_lds<f32x4>(ax);
             const f32x4 xb = lire_lds<f32x4>(ax + 64u);
-            if (((m + 1u) & 15u) == 0u && m + 1u < (TOUS ? nb_min : nb)) stager(m + 1u);
+            // the half's own tile goes on (the other one may end with this macro-step)
+            if (((m + 1u) & 15u) == 0u && m + 1u < nb) stager(m + 1u);
             ent_suiv = lire_lds<uint32_t>(a_ent_q + 32u * ((m + 1u) & 15u));
             const uint32_t lt = a_lut + (ent & ENT_CTX);
             uint32_t compte = 0;
