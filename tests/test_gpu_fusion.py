@@ -15,7 +15,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 import oracle_ffi as O  # noqa: E402
-from gpu_outils import Expert, dev, hote, vue, zeros  # noqa: E402
+from gpu_outils import Expert, dev, hote, mlp_f64, poids_f64, vue, zeros  # noqa: E402
 from troncons_amd import codeur, fusion  # noqa: E402
 from troncons_amd import noyaux as K  # noqa: E402
 from troncons_amd.noyaux import DimsExpert  # noqa: E402
@@ -158,6 +158,22 @@ def test_fused_gemv_small_shapes_and_break(fz, N):
     p[0] ^= 0xFF
     _, ctl = _gemv(fz, bytes(p), ex.luts, 1, 300, 256, O.synth_normale_bf16(5, 2, 1, 256, 1.0), *N)
     assert ctl[1] > 0
+
+
+@pytest.mark.parametrize("R,N", [(48, (4, 32)), (80, (4, 64)), (352, (16, 256))])
+def test_fused_gemv_pair_whose_second_tile_ends_on_a_group(fz, R, N):
+    """The last tile of a stream 16 or more whole macro-steps long and shorter than its pair's first: the
+    first one's entries of its next 16 macro-steps must still be staged (256 columns: a macro-step
+    per row)."""
+    dims = DimsExpert.de([R] * 3, [256] * 3)
+    ex = Expert(2031, dims, N_delta=N[0], N_codes=N[1])
+    x = O.synth_normale_bf16(2031, 1, 0, 256, 1.0)
+    p, l, y, ctl = dev(ex.partie), dev(ex.luts), zeros(4 * R), zeros(16)
+    tr = zeros(fusion.taille_travail_gemv(R, 256, 127))  # the fused form's workspace
+    fz.gemv_fusionnee(vue(p), 0, vue(l), R, 256, vue(dev(x)), vue(y), vue(ctl), vue(tr), *N)
+    y64 = O.gemv_mxfp4_f64(ex.attendu[:O.disposition_j([R] * 3, [256] * 3, 0).pas], x, R, 256)
+    assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
+    assert np.abs(hote(y, np.float32) - y64).max() <= TOL * np.abs(y64).max()
 
 
 def test_fused_gemv_wide_rows(fz):
@@ -435,3 +451,59 @@ def test_mount_counts_bad_parts(fz):
     bon = hote(rep, np.uint32).reshape(E * 3, 32)[:, 24]
     assert list(bon) == [1, 1, 1, 0, 0, 0, 0, 1, 1]
     couche.liberer()
+
+
+@pytest.mark.parametrize("N", [(64, 127), (1, 128), (63, 128), (256, 256), (300, 1000)])
+@pytest.mark.parametrize("d,r", [(256, 352), (2880, 288), (3072, 256), (3104, 256)])
+def test_long_tiles_layer_expert_and_gemv(fz, N, d, r):
+    """Tile lengths around 128, from which the selected matrices are decoded into workspace slots, and
+    row widths around the 3072 columns that the slots' GEMV takes: the layer step, one expert and one
+    matrix against f64 from the uncompressed weights; then the layer with only the fused form's
+    workspace (what a query for tiles of 127 returns), which gives the same within both forms'
+    tolerance; then with a selected expert's part damaged, which leaves the residual alone and counts
+    the same format errors in both forms."""
+    print(f"long tiles N {N} d {d} r {r}", flush=True)
+    E, k = 5, 3
+    dims = DimsExpert.de([r, r, d], [d, d, r])
+    experts = [codeur.synth_expert(41, 0, e, dims) for e in range(E)]
+    freqs = [codeur.tables([x[0][j] for x in experts], dims.lignes[j], dims.colonnes[j] // 32) for j in range(3)]
+    luts = dev(O.luts_couche([[freqs[j][t] for t in range(4)] for j in range(3)]))
+    octets = [codeur.partie(x[0], x[1], freqs, dims, expert=e, N_delta=N[0], N_codes=N[1])[0]
+              for e, x in enumerate(experts)]
+    routeur = np.stack([O.synth_normale_bf16(41, 3, e, d, 0.02) for e in range(E)])
+    r16, x = dev((routeur.view(np.uint32) >> 16).astype(np.uint16)), O.synth_normale_bf16(41, 4, 0, d, 1.0)
+    avant = O.synth_normale_bf16(41, 5, 0, d, 1.0)
+    oi, ow = O.routeur_topk(O.gemv_f32(routeur, x), k)
+    mlp = [mlp_f64(*experts[e], x.astype(np.float64)[:, None])[:, 0] for e in range(E)]
+    somme = sum(float(ow[i]) * mlp[e] for i, e in enumerate(oi))
+
+    def couche(parts, taille):
+        table = dev(np.array([p.data_ptr() for p in parts], np.uint64))
+        rep, ctl0, res, idx, w, ctl = zeros(fusion.taille_repertoire(E)), zeros(16), dev(avant), zeros(32), zeros(32), zeros(16)
+        fz.monter_couche(vue(table), E, dims, vue(rep), vue(ctl0))
+        tr = dev(np.full(taille, 0xFF, np.uint8))
+        fz.couche_moe(vue(rep), E, vue(luts), dims, vue(r16), None, vue(dev(x)), k, vue(res), vue(idx), vue(w),
+                      vue(ctl), vue(tr), *N)
+        assert (hote(idx, np.uint32)[:k] == oi).all() and np.abs(hote(w, np.float32)[:k] - ow).max() <= 1e-6
+        return hote(res, np.float32), list(hote(ctl, np.uint32))
+
+    parts = [dev(p) for p in octets]
+    tailles = (fusion.taille_travail_couche(dims, E, k, N[1]), fusion.taille_travail_couche(dims, E, k, 127))
+    for t in tailles:
+        got, ctl = couche(parts, t)
+        assert ctl == [0, 0, 0, 0]
+        assert np.abs(got - (avant + somme)).max() <= TOL * np.abs(avant + somme).max(), t
+    e0 = int(oi[1])
+    s, ctl = zeros(4 * d), zeros(16)
+    tr = zeros(fusion.taille_travail_expert(dims, N[1]))
+    fz.expert_fusionne(vue(parts[e0]), vue(luts), dims, vue(dev(x)), vue(s), vue(ctl), vue(tr), *N)
+    assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
+    assert np.abs(hote(s, np.float32) - mlp[e0]).max() <= TOL * np.abs(mlp[e0]).max()
+    y, ctl = _gemv(fz, octets[e0], hote(luts), 1, r, d, x, *N)
+    y64 = poids_f64(experts[e0][0][1], r, d) @ x.astype(np.float64) + experts[e0][1][1]
+    assert list(ctl) == [0, 0, 0, 0] and np.abs(y - y64).max() <= TOL * np.abs(y64).max()
+    casse = bytearray(octets[e0])
+    casse[0] ^= 1
+    vus = [couche([dev(bytes(casse)) if e == e0 else p for e, p in enumerate(parts)], t) for t in tailles]
+    assert (vus[0][0].view(np.uint32) == avant.view(np.uint32)).all()
+    assert vus[0][1] == vus[1][1] and vus[0][1][1] == 6 and vus[0][1][0] == vus[0][1][2] == 0

@@ -10,6 +10,8 @@
 //   fusion_codes     (N_codes 16, N_delta 1 or 2) the CODES pass decoding each tile's DELTA itself;
 //                    fusion_codes_swiglu, its MoE down form, builds its x (the SwiGLU row) itself;
 //   fusion_finir_combiner  the same for the k down products, then the weighted combine;
+//   fusion_longues_* (long tiles) the selected matrices decoded into workspace slots, then GEMVs over
+//                    the slots and the combine;
 //   fusion_routeur   (MoE layer) router logits; the first pass after it runs the top-k, and every
 //                    later kernel derives its jobs on the device from the chosen indices.
 //
@@ -31,8 +33,10 @@
 #include "chrono.hpp"
 #include "codes.hpp"
 #include "commun.hpp"
+#include "emplacement.hpp"
 #include "erreurs.hpp"
 #include "fusion_corps.hpp"
+#include "gemv.hpp"
 #include "selection.hpp"
 #include "norme.hpp"
 #include "passe.hpp"
@@ -587,6 +591,177 @@ fusion_finir_combiner(trc::Taches taches) {
                     moe.lignes[2], blockIdx.x * 256u + threadIdx.x, gridDim.x * 256u);
 }
 
+// ------------------------------------------------------------------------------------ long tiles
+// Streams of tiles of CHAINE_N_MIN macro-steps and more (the reference encoder writes 256): a matrix has
+// too few tiles to fill the chip, and a launch that decodes some of the matrices takes as long as one
+// that decodes them all, the length of one tile's chain of dependent steps. So every selected matrix is
+// decoded at once into a slot of the workspace, DELTA then CODES_CTX (down's with gate's and up's,
+// where the fused form must decode down after the SwiGLU), and the products are GEMVs over the slots.
+// Measured for a top-4 gpt-oss layer at 256/256: 612 -> 262 us (DELTA pass 308, gate/up 143 and down 141 us one
+// after the other before; DELTA 97, CODES_CTX 147, the GEMVs 10 and 8 now).
+struct Longues {
+    trc::Taches taches;      // TACHES_MOE_DELTA (job y = expert y / 3, matrix y % 3) or local jobs
+    uint64_t emplacements;   // slot of selected expert 0
+    uint64_t pas;            // bytes per slot
+    uint64_t etats;          // u32[jobs]: 1 once the job's matrix is decoded, 0 if it failed its checks
+    uint64_t produits;       // f32[k][3][rangs]: W x + b of gate and up, then of down
+    uint32_t rangs;          // rows per product
+    trc_dims_expert dims;    // of a whole expert (the matrices' places in its slot)
+};
+
+namespace trc {
+struct TravailLong {
+    uint32_t i, j;  // selected expert, matrix
+    uint32_t R, C;
+    trc_disposition disp;
+    uint8_t* mat;  // the matrix in its slot
+};
+__device__ __forceinline__ TravailLong travail_long(const Longues& p, uint32_t y) {
+    TravailLong t;
+    const bool local = p.taches.mode == TACHES_LOCALES;
+    t.i = local ? 0u : y / 3u;
+    t.j = local ? min(uniforme32(p.taches.locales[y].j), 2u) : y - 3u * t.i;
+    t.R = choisir(p.dims.lignes, t.j);
+    t.C = choisir(p.dims.colonnes, t.j);
+    t.disp = disposition(p.dims, t.j);
+    t.mat = reinterpret_cast<uint8_t*>(p.emplacements + uint64_t(t.i) * p.pas + t.disp.base);
+    return t;
+}
+// The checks of the fused passes (preparer_gemv): the job's streams are decoded only if they hold.
+__device__ __forceinline__ bool bon_long(const MatricePartie& m, const TravailLong& t, uint32_t kmax) {
+    const uint32_t B = t.C / 32u;
+    return m.bon != 0 && t.C % 32u == 0 && B >= 8u && t.R > 0 && (B - 1u) / (8u * m.cN) + 2u <= kmax;
+}
+}  // namespace trc
+
+// DELTA -> the slot's scales and biases. In a MoE layer every block runs the top-k first, as
+// fusion_echelles does; block (0, 0) publishes the selection, block (0, y) the job's record.
+extern "C" __global__ void __launch_bounds__(trc::FILS_ECHELLES)
+fusion_longues_echelles(Longues p, const uint32_t* __restrict__ luts, uint32_t* __restrict__ controle) {
+    using namespace trc;
+    __shared__ LdsEchelles<FILS_ECHELLES> s;
+    __shared__ uint32_t choisis[TOPK_MAX];
+    __shared__ __attribute__((aligned(16))) float lg[EXPERTS_MAX];
+    const TravailLong t = travail_long(p, blockIdx.y);
+    Tache tc;
+    if (p.taches.mode == TACHES_MOE_DELTA) {
+        const ParamsMoe& pm = p.taches.moe;
+        const gptr<float> logits = glob<float>(reinterpret_cast<const void*>(pm.logits));
+        for (uint32_t e = threadIdx.x; e < pm.E; e += FILS_ECHELLES) lg[e] = logits[e];
+        if (threadIdx.x < TOPK_MAX) choisis[threadIdx.x] = 0xFFFFFFFFu;
+        __syncthreads();
+        choisir_topk(lg, pm.E, pm.k, choisis, FILS_ECHELLES);
+        __syncthreads();
+        if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64u) {
+            float w[TOPK_MAX];
+            poids_topk(lg, choisis, pm.k, w);
+            if (threadIdx.x < pm.k) {
+                float wr = w[0];
+#pragma unroll
+                for (uint32_t r = 1; r < TOPK_MAX; ++r) wr = threadIdx.x == r ? w[r] : wr;
+                reinterpret_cast<uint32_t*>(pm.indices)[threadIdx.x] = choisis[threadIdx.x];
+                reinterpret_cast<float*>(pm.poids)[threadIdx.x] = wr;
+            }
+        }
+        tc = uniforme(tache_moe_e(pm, t.i, t.j, choisis[t.i]));
+    } else {
+        tc = uniforme(p.taches.locales[blockIdx.y]);
+    }
+    MatricePartie m;
+    if (p.taches.mode == TACHES_MOE_DELTA && tc.matrice == 0)  // the top-k left this place empty
+        m.bon = 0;
+    else
+        m = obtenir_matrice(tc);
+    const bool bon = bon_long(m, t, tc.kmax);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        reinterpret_cast<uint32_t*>(p.etats)[blockIdx.y] = bon ? 1u : 0u;
+        if (p.taches.mode == TACHES_MOE_DELTA && bon)
+            ecrire_matrice(reinterpret_cast<void*>(p.taches.moe.resolus + uint64_t(blockIdx.y) * sizeof(MatricePartie)), m);
+        if (!bon) atomicAdd(&controle[CTL_FORMAT], 1u);
+    }
+    if (!bon) return;
+    echelles_vers_emplacement<FILS_ECHELLES>(m.delta, m.med, m.biais, entete_de(m.delta, m.dP, m.dN, m.dT, m.dW), t.R,
+                                             t.C / 32u, t.mat, t.disp, luts + uint64_t(t.j) * 4u * M, controle, s);
+}
+
+// CODES_CTX -> the slot's code bytes.
+extern "C" __global__ void __launch_bounds__(trc::FILS_CODES_SLOT)
+fusion_longues_codes(Longues p, const uint32_t* __restrict__ luts, uint32_t* __restrict__ controle) {
+    using namespace trc;
+    __shared__ LdsCodes s;
+    const TravailLong t = travail_long(p, blockIdx.y);
+    if (reinterpret_cast<const uint32_t*>(p.etats)[blockIdx.y] == 0u) {  // counted once by each decoding launch
+        if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(&controle[CTL_FORMAT], 1u);
+        return;
+    }
+    MatricePartie m;
+    if (p.taches.mode == TACHES_MOE_DELTA)
+        m = lire_matrice_constante(p.taches.moe.resolus + uint64_t(blockIdx.y) * sizeof(MatricePartie));
+    else
+        m = obtenir_matrice(uniforme(p.taches.locales[blockIdx.y]));
+    codes_vers_emplacement<FILS_CODES_SLOT>(m.codes, m.med, entete_de(m.codes, m.cP, m.cN, m.cT, m.cW), t.R, t.C / 32u,
+                                            t.mat, t.disp, luts + (uint64_t(t.j) * 4u + 1u) * M, controle, s);
+}
+
+// y = W x + b over the slots. BAS: down of expert blockIdx.y, x its SwiGLU row, computed where x is
+// staged; otherwise job blockIdx.y of gate and up (or the one local job). The product goes to
+// `sortie` when there is one and else to its place in p.produits; nothing is written for an expert
+// with a matrix that failed its checks.
+namespace trc {
+struct XSwiglu {
+    gptr<f32x4> g4, u4;
+    __device__ __forceinline__ f32x4 operator()(uint32_t c) const {
+        const f32x4 g = g4[c], u = u4[c];
+        return f32x4{swiglu_oai_f(g.x, u.x), swiglu_oai_f(g.y, u.y), swiglu_oai_f(g.z, u.z), swiglu_oai_f(g.w, u.w)};
+    }
+};
+constexpr uint32_t FILS_GEMV_LONG = 512;
+}  // namespace trc
+template <bool BAS>
+__global__ void __launch_bounds__(trc::FILS_GEMV_LONG)
+fusion_longues_gemv(Longues p, const float* __restrict__ x, float* __restrict__ sortie) {
+    using namespace trc;
+    using F = FormeGemvX<FILS_GEMV_LONG, 1>;
+    __shared__ __attribute__((aligned(16))) uint8_t xl[F::LDS];
+    const bool local = p.taches.mode == TACHES_LOCALES;
+    const uint32_t i = BAS ? blockIdx.y : (local ? 0u : blockIdx.y >> 1);
+    const uint32_t y = BAS ? 3u * i + 2u : (local ? blockIdx.y : 3u * i + (blockIdx.y & 1u));
+    const TravailLong t = travail_long(p, y);
+    const uint32_t* etats = reinterpret_cast<const uint32_t*>(p.etats);
+    const bool bon = BAS ? etats[3u * i] != 0u && etats[3u * i + 1u] != 0u && etats[y] != 0u : etats[y] != 0u;
+    const uint32_t r_bloc = blockIdx.x * F::LIGNES;
+    if (!bon || r_bloc >= t.R) return;
+    float* produits = reinterpret_cast<float*>(p.produits) + uint64_t(3u * t.i) * p.rangs;
+    float* yy = sortie != nullptr ? sortie : produits + uint64_t(t.j) * p.rangs;
+    if (BAS)
+        gemv_mxfp4_x_lds<FILS_GEMV_LONG, 1>(t.mat, XSwiglu{glob<f32x4>(produits), glob<f32x4>(produits + p.rangs)}, yy,
+                                            t.R, t.C, r_bloc, xl);
+    else
+        gemv_mxfp4_x_lds<FILS_GEMV_LONG, 1>(t.mat, XCarte{glob<f32x4>(x)}, yy, t.R, t.C, r_bloc, xl);
+}
+
+// residu[r] += ((w0 s0[r] + w1 s1[r]) + ...) over the k down products, each product and sum rounded on
+// its own; nothing if a selected matrix failed its checks.
+extern "C" __global__ void __launch_bounds__(256) fusion_longues_combiner(Longues p) {
+#pragma clang fp contract(off)
+    using namespace trc;
+    const ParamsMoe& pm = p.taches.moe;
+    const uint32_t* etats = reinterpret_cast<const uint32_t*>(p.etats);
+    bool ok = true;
+    for (uint32_t y = 0; y < 3u * pm.k; ++y) ok = ok && etats[y] != 0u;
+    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
+    if (!ok || r >= p.dims.lignes[2]) return;
+    const gptr<float> bas = glob<float>(reinterpret_cast<const float*>(p.produits) + 2ull * p.rangs);
+    const gptr<float> poids = glob<float>(reinterpret_cast<const void*>(pm.poids));
+    float s = 0.0f;
+    for (uint32_t i = 0; i < pm.k; ++i) {
+        const float pr = poids[i] * bas[uint64_t(3u * i) * p.rangs + r];
+        s = i == 0 ? pr : s + pr;
+    }
+    float* residu = reinterpret_cast<float*>(pm.residu);
+    residu[r] = residu[r] + s;
+}
+
 // ---------------------------------------------------------------------------- router + top-k
 // Router logits y = W x (+ b), W bf16 row-major (E x C), in the reference gemv_f32 order (bf16 ->
 // f32 is exact, so the bits equal gemv_f32 on the widened matrix, passe.cuh:104-130): one row per
@@ -707,6 +882,9 @@ uint32_t kmax_pour(uint32_t colonnes, uint32_t n_codes) {
 
 uint64_t al(uint64_t x) { return (x + 255u) & ~uint64_t(255); }
 
+constexpr uint32_t LONGUES_N_MIN = 128;       // macro-steps per CODES_CTX tile from which tiles are long
+constexpr uint64_t LONGUES_TUILES = 8u * 256u;  // CODES_CTX tiles that one round of the decoding blocks takes
+
 uint32_t grille_tuiles(uint64_t octets, uint32_t N, uint32_t tuiles_par_bloc) {
     const uint64_t macro = (octets + 127) / 128;
     const uint64_t T = (macro + N - 1) / N;
@@ -741,6 +919,54 @@ uint64_t pas_tache(uint32_t R, uint32_t C, uint32_t n_codes) {
 // entries. In that plan each matrix may take either form (the kernels read N from its streams).
 // Other tile lengths take the DELTA pass, whose block entries go through the workspace.
 bool delta_interne(uint32_t n_delta, uint32_t n_codes) { return trc::delta_dans_codes(n_delta, n_codes); }
+
+// Long tiles (fusion_longues_*): decoded into workspace slots. From 128 macro-steps per CODES_CTX tile (254
+// tiles in a 2880 x 2880 matrix) and rows that the GEMV stages in LDS; and where the launches' length is
+// a chain's: DELTA tiles that are decoded as chains, or all CODES_CTX tiles in one round of blocks.
+// Measured, us for a gpt-oss layer step, slots / fused, by k and delta/codes tiles: 4 256/256 262 / 608,
+// 8 256/256 408 / 613, 1 256/256 251 / 598, 4 128/128 232 / 342, 8 128/128 318 / 348, 4 16/128 201 / 211;
+// shorter tiles: 4 64/64 176 / 179, 4 16/64 166 / 126.
+bool longues_possibles(uint32_t n_codes, uint32_t colonnes_max) {
+    return n_codes >= LONGUES_N_MIN && colonnes_max <= trc::GEMV_X_COLONNES;
+}
+bool longues(uint32_t R, uint32_t C, uint32_t jobs, uint32_t n_delta, uint32_t n_codes) {
+    if (!longues_possibles(n_codes, C)) return false;
+    return n_delta >= trc::CHAINE_N_MIN ||
+           uint64_t(jobs) * grille_tuiles(16ull * R * (C / 32u), n_codes, 1) <= LONGUES_TUILES;
+}
+// Workspace of `experts` experts' long tiles: states of their jobs, products, slots. rangs: rows per
+// product, a multiple of 64 floats.
+uint64_t octets_longues(const trc_dims_expert& dims, uint32_t experts, uint32_t* rangs) {
+    const uint32_t r = (std::max(dims.lignes[0], dims.lignes[2]) + 63u) / 64u * 64u;
+    if (rangs) *rangs = r;
+    return al(12ull * experts) + al(12ull * experts * r) + uint64_t(experts) * trc_taille_emplacement(&dims);
+}
+Longues par_longues(const Taches& t, const trc_dims_expert& dims, uint32_t experts, uint64_t base) {
+    Longues l;
+    std::memset(&l, 0, sizeof(l));
+    l.taches = t;
+    l.dims = dims;
+    octets_longues(dims, experts, &l.rangs);
+    l.etats = base;
+    l.produits = l.etats + al(12ull * experts);
+    l.emplacements = l.produits + al(12ull * experts * l.rangs);
+    l.pas = trc_taille_emplacement(&dims);
+    return l;
+}
+// Decoding launches of `jobs` matrices of at most R x C.
+int lancer_longues(const Longues& p, uint32_t R, uint32_t C, uint32_t jobs, uint32_t n_delta, uint32_t n_codes,
+                   const uint32_t* l, uint32_t* ctl, hipStream_t f) {
+    const uint64_t blocs = uint64_t(R) * (C / 32u);
+    TRC_LANCER(fusion_longues_echelles, dim3(grille_tuiles(blocs, n_delta, trc::TUILES_BLOC_ECHELLES), jobs),
+               dim3(trc::FILS_ECHELLES), f, p, l, ctl);
+    TRC_LANCER(fusion_longues_codes, dim3(grille_tuiles(16u * blocs, n_codes, trc::TUILES_BLOC_CODES), jobs),
+               dim3(trc::FILS_CODES_SLOT), f, p, l, ctl);
+    return TRC_OK;
+}
+dim3 grille_gemv_long(uint32_t lignes, uint32_t jobs) {
+    constexpr uint32_t L = trc::FormeGemvX<trc::FILS_GEMV_LONG, 1>::LIGNES;
+    return dim3((lignes + L - 1u) / L, jobs);
+}
 
 // Workspace piece of one matrix job in the internal-DELTA mode: its partial sums only.
 uint64_t pas_tache_interne(uint32_t R, uint32_t C) { return al(4ull * R * kmax_pour(C, 16)); }
@@ -822,9 +1048,24 @@ int lancer_echelles_prefill(const ParamsMoe& pm, uint32_t R, uint32_t C, uint32_
 uint64_t octets_entrees(uint32_t R, uint32_t C) { return octets_ech(R, C); }
 }  // namespace trc
 
-extern "C" uint64_t trc_taille_travail_gemv_fusionnee(uint32_t lignes, uint32_t colonnes, uint32_t n_codes) {
+// The workspace sizes: what the fused form needs (accepted whatever the tile length), and what the
+// queries return, which for long tiles also covers the slots of fusion_longues_*. A call whose
+// workspace does not cover them takes the fused form.
+namespace {
+uint64_t travail_gemv_min(uint32_t lignes, uint32_t colonnes, uint32_t n_codes) {
     if (colonnes / 32 < 8 || n_codes == 0) return 0;
     return pas_tache(lignes, colonnes, n_codes);
+}
+// One matrix as the expert whose three matrices it is (only its own place is used).
+trc_dims_expert dims_matrice(uint32_t lignes, uint32_t colonnes) {
+    return trc_dims_expert{{lignes, lignes, lignes}, {colonnes, colonnes, colonnes}};
+}
+}  // namespace
+
+extern "C" uint64_t trc_taille_travail_gemv_fusionnee(uint32_t lignes, uint32_t colonnes, uint32_t n_codes) {
+    const uint64_t m = travail_gemv_min(lignes, colonnes, n_codes);
+    if (m == 0 || !longues_possibles(n_codes, colonnes)) return m;
+    return std::max(m, octets_longues(dims_matrice(lignes, colonnes), 1, nullptr));
 }
 
 // Config 1: one matrix j of a part, y = W_j x + b_j, decoded in registers.
@@ -840,7 +1081,7 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
     TRC_VERIFIER(x.adresse && x.octets >= 4ull * colonnes && x.adresse % 16 == 0, "x trop court ou non aligne");
     TRC_VERIFIER(y.adresse && y.octets >= 4ull * lignes, "y trop court");
     TRC_VERIFIER(controle.adresse && controle.octets >= 16, "controle de moins de 16 o");
-    const uint64_t besoin = trc_taille_travail_gemv_fusionnee(lignes, colonnes, n_codes);
+    const uint64_t besoin = travail_gemv_min(lignes, colonnes, n_codes);
     TRC_VERIFIER(travail.adresse && travail.octets >= besoin && travail.adresse % 256 == 0,
                  "travail de %llu o, %llu o demandes (aligne sur 256)", (unsigned long long)travail.octets,
                  (unsigned long long)besoin);
@@ -867,6 +1108,15 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
         return TRC_OK;
     }
     const Taches tv = par_valeur(&t, 1);
+    if (longues(lignes, colonnes, 1, n_delta, n_codes) &&
+        travail.octets >= trc_taille_travail_gemv_fusionnee(lignes, colonnes, n_codes)) {
+        const Longues p = par_longues(tv, dims_matrice(lignes, colonnes), 1, travail.adresse);
+        const int r = lancer_longues(p, lignes, colonnes, 1, n_delta, n_codes, l, ctl, f);
+        if (r != TRC_OK) return r;
+        TRC_LANCER(fusion_longues_gemv<false>, grille_gemv_long(lignes, 1), dim3(trc::FILS_GEMV_LONG), f, p,
+                   reinterpret_cast<const float*>(x.adresse), reinterpret_cast<float*>(y.adresse));
+        return TRC_OK;
+    }
     TRC_LANCER(fusion_echelles, dim3(grille_echelles(uint64_t(lignes) * B, n_delta, 1), 1),
                dim3(trc::FILS_ECHELLES_FUSION), f, tv, l, ctl);
     TRC_LANCER_GEMV("fusion_gemv", forme_gemv(lignes, colonnes, n_codes, 1), f, tv, l, ctl);
@@ -874,12 +1124,20 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
     return TRC_OK;
 }
 
-extern "C" uint64_t trc_taille_travail_expert_fusionne(const trc_dims_expert* dims, uint32_t n_codes) {
+namespace {
+uint64_t travail_expert_min(const trc_dims_expert* dims, uint32_t n_codes) {
     if (verifier_forme(dims, n_codes) != TRC_OK) return 0;
     const uint32_t R = dims->lignes[0], C = dims->colonnes[0];
     const uint32_t Rm = dims->lignes[2] > R ? dims->lignes[2] : R;
     const uint32_t Cm = dims->colonnes[2] > C ? dims->colonnes[2] : C;
     return 3 * pas_tache(Rm, Cm, n_codes) + al(4ull * R);
+}
+}  // namespace
+
+extern "C" uint64_t trc_taille_travail_expert_fusionne(const trc_dims_expert* dims, uint32_t n_codes) {
+    const uint64_t m = travail_expert_min(dims, n_codes);
+    if (m == 0 || !longues_possibles(n_codes, std::max(dims->colonnes[0], dims->colonnes[2]))) return m;
+    return std::max(m, octets_longues(*dims, 1, nullptr));
 }
 
 // Config 2: one expert, s = W_down swiglu(W_gate x + b_gate, W_up x + b_up) + b_down, every matrix
@@ -899,7 +1157,7 @@ extern "C" int trc_expert_fusionne(trc_vue partie, trc_vue luts, const trc_dims_
     TRC_VERIFIER(x.adresse && x.octets >= 4ull * C && x.adresse % 16 == 0, "x trop court ou non aligne");
     TRC_VERIFIER(sortie.adresse && sortie.octets >= 4ull * dims->lignes[2], "sortie trop courte");
     TRC_VERIFIER(controle.adresse && controle.octets >= 16, "controle de moins de 16 o");
-    const uint64_t besoin = trc_taille_travail_expert_fusionne(dims, n_codes);
+    const uint64_t besoin = travail_expert_min(dims, n_codes);
     TRC_VERIFIER(travail.adresse && travail.octets >= besoin && travail.adresse % 256 == 0,
                  "travail de %llu o, %llu o demandes (aligne sur 256)", (unsigned long long)travail.octets,
                  (unsigned long long)besoin);
@@ -940,6 +1198,16 @@ extern "C" int trc_expert_fusionne(trc_vue partie, trc_vue luts, const trc_dims_
         return TRC_OK;
     }
     const Taches trois = par_valeur(t, 3), bas = par_valeur(t + 2, 1);
+    if (longues(Rm, Cm, 3, n_delta, n_codes) && travail.octets >= trc_taille_travail_expert_fusionne(dims, n_codes)) {
+        const Longues p = par_longues(trois, *dims, 1, base);
+        r = lancer_longues(p, Rm, Cm, 3, n_delta, n_codes, l, ctl, f);
+        if (r != TRC_OK) return r;
+        TRC_LANCER(fusion_longues_gemv<false>, grille_gemv_long(R, 2), dim3(trc::FILS_GEMV_LONG), f, p,
+                   reinterpret_cast<const float*>(x.adresse), static_cast<float*>(nullptr));
+        TRC_LANCER(fusion_longues_gemv<true>, grille_gemv_long(dims->lignes[2], 1), dim3(trc::FILS_GEMV_LONG), f, p,
+                   static_cast<const float*>(nullptr), reinterpret_cast<float*>(sortie.adresse));
+        return TRC_OK;
+    }
     TRC_LANCER(fusion_echelles, dim3(grille_echelles(uint64_t(Rm) * (Cm / 32), n_delta, 3), 3),
                dim3(trc::FILS_ECHELLES_FUSION), f, trois, l, ctl);
     TRC_LANCER_GEMV("fusion_gemv", forme_gemv(R, C, n_codes, 2), f, trois, l, ctl);
@@ -975,14 +1243,30 @@ extern "C" int trc_monter_couche(trc_vue parties, uint32_t experts, const trc_di
     return TRC_OK;
 }
 
-extern "C" uint64_t trc_taille_travail_couche_moe(const trc_dims_expert* dims, uint32_t experts, uint32_t k,
-                                                  uint32_t n_codes) {
+namespace {
+// The part of a layer's workspace before its jobs' pieces.
+uint64_t travail_couche_tete(const trc_dims_expert& dims, uint32_t experts, uint32_t k) {
+    return al(4ull * experts) + al(3ull * k * sizeof(trc::MatricePartie)) + al(4ull * k * dims.lignes[0]) +
+           al(12ull * k * std::max(dims.lignes[0], dims.lignes[2]));
+}
+uint64_t travail_couche_min(const trc_dims_expert* dims, uint32_t experts, uint32_t k, uint32_t n_codes) {
     if (verifier_forme(dims, n_codes) != TRC_OK || k == 0 || k > trc::TOPK_MAX || experts == 0) return 0;
     const uint32_t R = dims->lignes[0], C = dims->colonnes[0];
     const uint32_t Rm = dims->lignes[2] > R ? dims->lignes[2] : R;
     const uint32_t Cm = dims->colonnes[2] > C ? dims->colonnes[2] : C;
-    return al(4ull * experts) + al(3ull * k * sizeof(trc::MatricePartie)) + al(4ull * k * R) + al(12ull * k * Rm) +
-           3ull * k * pas_tache(Rm, Cm, n_codes);
+    return travail_couche_tete(*dims, experts, k) + 3ull * k * pas_tache(Rm, Cm, n_codes);
+}
+}  // namespace
+
+extern "C" uint64_t trc_taille_travail_couche_moe(const trc_dims_expert* dims, uint32_t experts, uint32_t k,
+                                                  uint32_t n_codes) {
+    const uint64_t m = travail_couche_min(dims, experts, k, n_codes);
+    if (m == 0 || !longues_possibles(n_codes, std::max(dims->colonnes[0], dims->colonnes[2]))) return m;
+    return std::max(m, travail_couche_tete(*dims, experts, k) + octets_longues(*dims, k, nullptr));
+}
+
+uint64_t trc::taille_travail_couche_min(const trc_dims_expert* dims, uint32_t experts, uint32_t k, uint32_t n_codes) {
+    return travail_couche_min(dims, experts, k, n_codes);
 }
 
 // Config 3: one MoE layer decode step at batch 1. logits = W_r x (+ b_r) (W_r bf16, experts x C),
@@ -1027,7 +1311,7 @@ int couche_moe(trc_vue repertoire, uint32_t experts, trc_vue luts, const trc_dim
     TRC_VERIFIER(indices.adresse && indices.octets >= 4ull * k && poids.adresse && poids.octets >= 4ull * k,
                  "indices ou poids trop courts");
     TRC_VERIFIER(controle.adresse && controle.octets >= 16, "controle de moins de 16 o");
-    const uint64_t besoin = trc_taille_travail_couche_moe(dims, experts, k, n_codes);
+    const uint64_t besoin = travail_couche_min(dims, experts, k, n_codes);
     TRC_VERIFIER(travail.adresse && travail.octets >= besoin && travail.adresse % 256 == 0,
                  "travail de %llu o, %llu o demandes (aligne sur 256)", (unsigned long long)travail.octets,
                  (unsigned long long)besoin);
@@ -1117,6 +1401,19 @@ int couche_moe(trc_vue repertoire, uint32_t experts, trc_vue luts, const trc_dim
         TRC_LANCER(fusion_finir_combiner, dim3((D + 255) / 256), dim3(256), f, t_bas);
         return TRC_OK;
     }
+    if (longues(Rm, std::max(C, R), 3 * k, n_delta, n_codes) &&
+        travail.octets >= trc_taille_travail_couche_moe(dims, experts, k, n_codes)) {
+        const Longues pl = par_longues(t_delta, *dims, k, morceaux);
+        r = lancer_longues(pl, Rm, std::max(C, R), 3 * k, n_delta, n_codes, l, ctl, f);
+        if (r != TRC_OK) return r;
+        TRC_LANCER_N("fusion_longues_gemv/gate_up", fusion_longues_gemv<false>, grille_gemv_long(R, 2 * k),
+                     dim3(trc::FILS_GEMV_LONG), f, pl, reinterpret_cast<const float*>(x.adresse),
+                     static_cast<float*>(nullptr));
+        TRC_LANCER_N("fusion_longues_gemv/down", fusion_longues_gemv<true>, grille_gemv_long(D, k),
+                     dim3(trc::FILS_GEMV_LONG), f, pl, static_cast<const float*>(nullptr), static_cast<float*>(nullptr));
+        TRC_LANCER(fusion_longues_combiner, dim3((D + 255) / 256), dim3(256), f, pl);
+        return TRC_OK;
+    }
     TRC_LANCER(fusion_echelles, dim3(grille_echelles(uint64_t(R) * (C / 32), n_delta, 3 * k), 3 * k),
                dim3(trc::FILS_ECHELLES_FUSION), f, t_delta, l, ctl);
     TRC_LANCER_N("fusion_gemv/gate_up", fusion_gemv, forme_gemv(R, C, n_codes, 2 * k).grille,
@@ -1196,7 +1493,7 @@ extern "C" int trc_couche_moe_fusionnee_sans_alloc(trc_vue repertoire, uint32_t 
                                                    trc_vue routeur_biais, trc_vue x, uint32_t k, trc_vue residu,
                                                    trc_vue indices, trc_vue poids, trc_vue controle, uint32_t n_delta,
                                                    uint32_t n_codes, void* flux) {
-    const uint64_t besoin = trc_taille_travail_couche_moe(dims, experts, k, n_codes);
+    const uint64_t besoin = travail_couche_min(dims, experts, k, n_codes);
     if (besoin == 0) return usage("forme, top-k ou N refuses");
     if (besoin > OCTETS_SCRATCH)
         return usage("l'etape demande %llu o de travail, la memoire statique en a %llu",

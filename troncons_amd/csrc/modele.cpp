@@ -47,9 +47,10 @@ uint64_t taille_moe(const trc_hyper& h) {
     return trc_taille_travail_couche_moe(&h.dims, h.experts, h.actifs, h.n_codes);
 }
 
-uint64_t taille_travail(const trc_hyper& h) {
+// Workspace bytes with `moe` of them for the MoE layers.
+uint64_t taille_travail(const trc_hyper& h, uint64_t moe) {
     const uint64_t d = h.d, dq = uint64_t(h.tetes) * 64, dkv = uint64_t(h.tetes_kv) * 64;
-    return al(4 * d) * 3 + al(4 * dq) * 2 + al(4 * dkv) * 2 + al(4 * d) + al(4 * 8) * 2 + al(16) + al(taille_moe(h)) +
+    return al(4 * d) * 3 + al(4 * dq) * 2 + al(4 * dkv) * 2 + al(4 * d) + al(4 * 8) * 2 + al(16) + al(moe) +
            al(4ull * h.vocab) + al(4) + al(16 * 32);
 }
 
@@ -72,7 +73,7 @@ int verifier_hyper(const trc_hyper* h) {
 
 extern "C" uint64_t trc_modele_taille_travail(const trc_hyper* h) {
     if (verifier_hyper(h) != TRC_OK) return 0;
-    return taille_travail(*h);
+    return taille_travail(*h, taille_moe(*h));
 }
 
 extern "C" int trc_modele_creer(const trc_hyper* h, const trc_couche_modele* couches, trc_vue enchassement,
@@ -82,7 +83,11 @@ extern "C" int trc_modele_creer(const trc_hyper* h, const trc_couche_modele* cou
     int r = verifier_hyper(h);
     if (r != TRC_OK) return r;
     if (couches == nullptr) return trc::usage("couches absentes");
-    const uint64_t besoin = taille_travail(*h);
+    // a workspace too small for the MoE layers' preferred form keeps the form that needs less
+    uint64_t moe = taille_moe(*h);
+    if (travail.octets < taille_travail(*h, moe))
+        moe = trc::taille_travail_couche_min(&h->dims, h->experts, h->actifs, h->n_codes);
+    const uint64_t besoin = taille_travail(*h, moe);
     TRC_VERIFIER(travail.adresse && travail.adresse % 256 == 0 && travail.octets >= besoin,
                  "travail de %llu o, %llu o demandes (aligne sur 256)", (unsigned long long)travail.octets,
                  (unsigned long long)besoin);
@@ -113,7 +118,7 @@ extern "C" int trc_modele_creer(const trc_hyper* h, const trc_couche_modele* cou
     n->idx = t.prendre(4 * 8);
     n->pw = t.prendre(4 * 8);
     n->controle = t.prendre(16);
-    n->moe = t.prendre(taille_moe(*h));
+    n->moe = t.prendre(moe);
     n->z = t.prendre(4ull * h->vocab);
     n->jeton = t.prendre(4);
     n->table = t.prendre(16 * 32);

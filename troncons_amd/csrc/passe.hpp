@@ -33,4 +33,8 @@ int lancer_couche_moe_normee(trc_vue repertoire, uint32_t experts, trc_vue luts,
                              trc_vue residu, trc_vue indices, trc_vue poids, trc_vue controle, trc_vue travail,
                              uint32_t n_delta, uint32_t n_codes, void* flux);
 
+// (fusion.hip) The smallest workspace that a MoE layer step accepts: below trc_taille_travail_couche_moe
+// for long tiles, which then take the form that decodes them where they are multiplied.
+uint64_t taille_travail_couche_min(const trc_dims_expert* dims, uint32_t experts, uint32_t k, uint32_t n_codes);
+
 }  // namespace trc
