@@ -401,7 +401,9 @@ __device__ __forceinline__ void corps_codes_n(const Tache& tc, const PrepCodes& 
         // 3. the CODES words over the DELTA ones, and the next pair's streams read ahead
         ecrire_lds<u32x4>(a_anneau + 16u * v, cur.mots0);
         ecrire_lds<u32x4>(a_anneau + 512u + 16u * v, cur.mots1);
-        av = lire_avance<true>(h, p.fc, hd, p.fd, p.med, R, p.B, t + 2u * n_vagues, v);
+        // (wave-uniform test: with one pair per wavefront, as in a top-4 gpt-oss layer, the unused
+        // read-ahead cost 0.8 of 54.5 us per step; the slot decoder, with several, is better without it)
+        if (t0 + 2u * n_vagues < hT) av = lire_avance<true>(h, p.fc, hd, p.fd, p.med, R, p.B, t + 2u * n_vagues, v);
         AnneauR a;
         {
             const uint32_t mot0 = mots_c + 2u * cur.tete.debut;
@@ -412,8 +414,9 @@ __device__ __forceinline__ void corps_codes_n(const Tache& tc, const PrepCodes& 
             a.o2 = mot0 - a.g0;
             a.charge = OCTETS_ANNEAU / OCTETS_MORCEAU;
             a.limite = a.charge * OCTETS_MORCEAU - FENETRE;
-            a.vol = u32x2{0u, 0u};
-            a.en_vol = false;
+            // the chunk in flight is chunk 3, which has landed with the others: its first landing is
+            // the same bytes again
+            a.vol = lire_lds<u32x2>(a_anneau + 768u + 8u * v);
         }
         uint32_t x = cur.tete.x;
         const uint32_t debut = cur.tete.debut, attendu = cur.tete.attendu;
@@ -633,8 +636,9 @@ __device__ __forceinline__ void corps_codes_emplacement_n(const PrepCodes& p, ui
             a.o2 = mot0 - a.g0;
             a.charge = OCTETS_ANNEAU / OCTETS_MORCEAU;
             a.limite = a.charge * OCTETS_MORCEAU - FENETRE;
-            a.vol = u32x2{0u, 0u};
-            a.en_vol = false;
+            // the chunk in flight is chunk 3, which has landed with the others: its first landing is
+            // the same bytes again
+            a.vol = lire_lds<u32x2>(a_anneau + 768u + 8u * v);
         }
         uint32_t x = cur.tete.x;
         const uint32_t debut = cur.tete.debut, attendu = cur.tete.attendu;

@@ -195,11 +195,26 @@ __device__ __forceinline__ void verser_controle(uint32_t* controle, uint32_t hor
     }
 }
 
-// 32-lane xor butterfly within each half-wavefront (the reference's warp reduction tree).
+// v of another lane of its row of 16, by a DPP control (no LDS round trip, unlike __shfl_xor).
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;                          // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int DPP_TOUR4 = 0x124, DPP_TOUR8 = 0x128, DPP_MIROIR8 = 0x141;  // row_ror 4 and 8, row_half_mirror
+template <int DPP>
+__device__ __forceinline__ float voisin(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP, 0xF, 0xF, false));
+}
+
+// 32-lane xor butterfly within each half-wavefront (the reference's warp reduction tree: lane distances
+// 16, 8, 4, 2, 1; every lane gets the same bits). Distance 16 by a swap of rows of 16, 8 by a rotation of
+// the row; once lanes 8 apart agree, a rotation by 4 reaches the lane at xor 4. All in registers: through
+// ds_bpermute the five levels took five LDS round trips (some 650 cycles), as long as half a macro-step
+// of the CODES pass, which closes a row in about every sixth one.
 __device__ __forceinline__ float somme_demi_f32(float v) {
-#pragma unroll
-    for (int d = 16; d > 0; d >>= 1) v += __shfl_xor(v, d);
-    return v;
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    v += voisin<DPP_TOUR8>(v);
+    v += voisin<DPP_TOUR4>(v);
+    v += voisin<DPP_XOR2>(v);
+    return v + voisin<DPP_XOR1>(v);
 }
 
 // 2^(e-128) in f32, exact for every e (e = 0, 1 are subnormal).

@@ -714,7 +714,14 @@ __device__ __forceinline__ void corps_gemv_xg(const Tache& tc, const PrepGemv& p
 // row. Stream padding blocks read the zero slot of x, so no per-block validity test is needed.
 
 // A tile's word ring (as Anneau, with absolute LDS addresses; `lds` is 1 KiB aligned). Chunks are
-// addressed by 32-bit offsets from the stream's start, which both tiles of a wavefront share.
+// addressed by 32-bit offsets from the stream's start, which both tiles of a wavefront share. One
+// chunk is always in flight: when the pointer passes into a chunk, the one in flight lands (two chunks
+// ahead of the pointer, so before any macro-step can read it) and the next is requested, into the slot of
+// the chunk just left. A chunk so has the time that 256 bytes of words last, two macro-steps or more
+// for MXFP4 codes, and at least one; a macro-step makes one test. (Landing each chunk one macro-step after
+// its request took a second test and waited for device memory: a 512-position prefill 807 -> 787 us, a
+// layer of 256-macro-step tiles 272 -> 261 us, one expert 52.3 -> 51.8 us, a top-4 layer step of one pair per
+// wavefront 53.8 -> 54.5 us.)
 struct AnneauR {
     const uint8_t* flux;  // start of the stream (its descriptor's p)
     uint32_t g0;      // offset from `flux` of the tile's 16-byte aligned word origin
@@ -723,8 +730,7 @@ struct AnneauR {
     uint32_t o2;      // byte offset from g0 of the next word (unwrapped)
     uint32_t limite;  // refill when o2 > limite (= charge * 256 - FENETRE)
     uint32_t charge;  // next chunk to request
-    u32x2 vol;
-    bool en_vol;
+    u32x2 vol;        // this lane's 8 bytes of chunk charge - 1, not yet in LDS
 };
 
 __device__ __forceinline__ u32x2 lire_morceau_r(const AnneauR& a, uint32_t c, uint32_t v) {
@@ -746,30 +752,23 @@ __device__ __forceinline__ AnneauR ouvrir_anneau_r(const EnteteRans& h, const De
     a.charge = OCTETS_ANNEAU / OCTETS_MORCEAU;
     a.limite = a.charge * OCTETS_MORCEAU - FENETRE;
     a.vol = u32x2{0u, 0u};
-    a.en_vol = false;
     if (tuile) {
-        const u32x2 d0 = lire_morceau_r(a, 0, v), d1 = lire_morceau_r(a, 1, v);
-        const u32x2 d2 = lire_morceau_r(a, 2, v), d3 = lire_morceau_r(a, 3, v);
+        const u32x2 d0 = lire_morceau_r(a, 0, v), d1 = lire_morceau_r(a, 1, v), d2 = lire_morceau_r(a, 2, v);
+        a.vol = lire_morceau_r(a, 3, v);
         ecrire_lds<u32x2>(lds + 0u * OCTETS_MORCEAU + v * 8u, d0);
         ecrire_lds<u32x2>(lds + 1u * OCTETS_MORCEAU + v * 8u, d1);
         ecrire_lds<u32x2>(lds + 2u * OCTETS_MORCEAU + v * 8u, d2);
-        ecrire_lds<u32x2>(lds + 3u * OCTETS_MORCEAU + v * 8u, d3);
     }
     return a;
 }
 
-// End of a macro-step: land the chunk requested one macro-step ago (chunk charge - 1), request the
-// next if due (the same schedule as avancer_anneau).
+// End of a macro-step: at most one chunk to land and one to request (a macro-step uses at most 256 bytes).
 __device__ __forceinline__ void avancer_anneau_r(AnneauR& a, uint32_t v, bool actif) {
-    if (a.en_vol) {
-        ecrire_lds<u32x2>(a.lds + ((a.charge - 1u) & 3u) * OCTETS_MORCEAU + v * 8u, a.vol);
-        a.en_vol = false;
-    }
     if (actif && a.o2 > a.limite) {
+        ecrire_lds<u32x2>(a.lds + ((a.charge - 1u) & 3u) * OCTETS_MORCEAU + v * 8u, a.vol);
         a.vol = lire_morceau_r(a, a.charge, v);
         a.charge += 1u;
         a.limite += OCTETS_MORCEAU;
-        a.en_vol = true;
     }
 }
 

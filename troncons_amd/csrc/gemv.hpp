@@ -18,21 +18,11 @@
 //          pairs at lane distance 16, then 8, 4, 2, 1 (every lane of the tree ends with the same S).
 // Mapping here: a 32-lane half-wavefront owns a row (l = its lane), two rows per half for MXFP4
 // (the x loads of a block serve both); E2M1 pairs are expanded by v_cvt_scalef32_pk_f32_fp4 (scale
-// 2: the doubled values); the tree runs on ds_swizzle (xor masks within 32 lanes); the loads of a
+// 2: the doubled values); the tree runs on DPP exchanges (somme_demi_f32); the loads of a
 // lane's next block are issued before the current block's arithmetic.
 namespace trc {
 
 constexpr uint32_t GEMV_LIGNES_PAR_DEMI = 2;
-
-// S: the xor tree over a half-wavefront's 32 lanes.
-__device__ __forceinline__ float arbre_32(float v) {
-    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));  // xor 16
-    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x201F));  // xor 8
-    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x101F));  // xor 4
-    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x081F));  // xor 2
-    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x041F));  // xor 1
-    return v;
-}
 
 // Bytes 4t .. 4t + 3 of a block (code word t) continuing the chain s: byte 4t + k pairs with
 // x[4t + k] (low nibble) and x[16 + 4t + k] (high nibble), i.e. xa[k] and xb[k].
@@ -102,7 +92,7 @@ __device__ __forceinline__ void gemv_mxfp4_demi(const uint8_t* __restrict__ mat,
     const gptr<float> biais = glob<float>(mat + d.biais);
 #pragma unroll
     for (uint32_t i = 0; i < GEMV_LIGNES_PAR_DEMI; ++i) {
-        const float s = arbre_32(acc[i]);
+        const float s = somme_demi_f32(acc[i]);
         if (l == 0u && r0 + i < R) y[r0 + i] = s + biais[r0 + i];
     }
 }
@@ -195,7 +185,7 @@ __device__ __forceinline__ void gemv_mxfp4_x_lds_n(const uint8_t* __restrict__ m
     const gptr<float> biais = glob<float>(mat + d.biais);
 #pragma unroll
     for (uint32_t i = 0; i < PD; ++i) {
-        const float s = arbre_32(acc[i]);
+        const float s = somme_demi_f32(acc[i]);
         if (l == 0u && r0 + i < R) y[r0 + i] = s + biais[r0 + i];
     }
 }

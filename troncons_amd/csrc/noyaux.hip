@@ -195,7 +195,7 @@ gemv_f32(const float* __restrict__ W, const float* __restrict__ x, const float* 
         acc = fmaf(w.z, xv.z, acc);
         acc = fmaf(w.w, xv.w, acc);
     }
-    const float s = arbre_32(acc);
+    const float s = somme_demi_f32(acc);
     if (l == 0u) y[r] = biais != nullptr ? s + biais[r] : s;
 }
 

@@ -475,12 +475,6 @@ __device__ __forceinline__ f32x8 lire_brut(const float* p) {
     return r;
 }
 
-// v of the lane at xor 1, at xor 2, mirrored within its eight lanes (quad_perm, row_half_mirror).
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_MIROIR8 = 0x141;
-template <int DPP>
-__device__ __forceinline__ float voisin(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), DPP, 0xF, 0xF, false));
-}
 // Sum and maximum over the eight lanes of a group; every lane gets the same bits.
 __device__ __forceinline__ float somme_groupe(float v) {
     v += voisin<DPP_XOR1>(v);
