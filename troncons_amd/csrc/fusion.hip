@@ -975,7 +975,9 @@ uint64_t pas_tache_interne(uint32_t R, uint32_t C) { return al(4ull * R * kmax_p
 // tiles) per block, the largest that still gives every CU of the chip a block, and at most about one
 // block per CU over all jobs (a block's LDS holds the three LUTs, so one fits a CU): wavefronts then
 // loop over further tile pairs instead of new blocks paying the LUT staging and the header reads.
-constexpr uint32_t CUS = 256;
+// "Every CU" up to a sixteenth: 254 blocks of 512 threads take gate and up of a gpt-oss expert at 16
+// macro-steps per tile in one round where 256 blocks of 256 threads need two (one expert: 51.8 -> 41.0 us).
+constexpr uint32_t CUS = 256, CUS_PRESQUE = CUS - CUS / 16u;
 
 struct FormeGemv {
     dim3 grille, bloc;
@@ -986,7 +988,7 @@ FormeGemv forme_gemv(uint32_t R, uint32_t C, uint32_t N, uint32_t jobs) {
     const uint64_t octets = 16ull * R * (C / 32);
     const uint64_t T = ((octets + 127) / 128 + N - 1) / N;
     uint32_t fils = trc::FILS_GEMV_MAX;
-    while (fils > 256 && ((T + fils / 32 - 1) / (fils / 32)) * jobs < CUS) fils /= 2;
+    while (fils > 256 && ((T + fils / 32 - 1) / (fils / 32)) * jobs < CUS_PRESQUE) fils /= 2;
     uint32_t gx = grille_tuiles(octets, N, fils / 32);
     const uint32_t plafond = (CUS + jobs - 1) / jobs;
     if (gx > plafond) gx = plafond;
