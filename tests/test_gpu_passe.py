@@ -58,6 +58,22 @@ def test_gemv_q8_0_bit_exact_against_oracle(k, r, c):
     assert (_q8(k, o, x, None, r, c).view(np.uint32) == O.gemv_q8_0(o, x, None, r, c).view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("r,c", [(33, 14560), (33, 14592), (32767, 96), (32768, 96), (32773, 352), (32769, 8192),
+                                 (32769, 8224)])
+def test_gemv_q8_0_at_the_limits_of_its_forms(k, r, c):
+    """Row counts around 32768 (one or four rows per half-wavefront) that do not fill a block, and widths
+    around those whose x each form stages in LDS: bit for bit equal to the oracle."""
+    print(f"gemv_q8_0 limits {r}x{c}", flush=True)
+    rng = np.random.default_rng(r + c)
+    o = np.empty((r * (c // 32), 34), np.uint8)
+    o[:, :2] = (rng.standard_normal(len(o), dtype=np.float32) * 0.01).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    o[:, 2:] = rng.integers(0, 256, size=(len(o), 32), dtype=np.uint8)
+    o = o.ravel()
+    x = rng.standard_normal(c).astype(np.float32)
+    b = rng.standard_normal(r).astype(np.float32)
+    assert (_q8(k, o, x, b, r, c).view(np.uint32) == O.gemv_q8_0(o, x, b, r, c).view(np.uint32)).all()
+
+
 def test_gemv_q8_0_unaligned_matrix_and_last_block(k):
     # a matrix starting 2 bytes past a 4-byte boundary (the contract allows any even address), with
     # the last block's window reaching past the matrix end on a view that ends there

@@ -33,8 +33,13 @@ __device__ __forceinline__ double somme_arbre_f64(double* part, double* total, d
 // in full before the first write (y may be x). Up to NORME_PAR_FIL * 256 elements a thread holds
 // its x and w values in registers, so all its loads go out together.
 constexpr uint32_t NORME_PAR_FIL = 16;
+// Where y_i goes: y + i.
+struct PlaceSuite {
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return i; }
+};
+template <class Place = PlaceSuite>
 __device__ __forceinline__ void norme_ligne(const float* __restrict__ x, const float* __restrict__ w, float* y,
-                                            uint32_t n, float eps, double* part, double* total) {
+                                            uint32_t n, float eps, double* part, double* total, Place place = {}) {
     const uint32_t t = threadIdx.x;
     if (n <= NORME_PAR_FIL * FILS_NORME) {
         // indices clamped to the row (no branch around a load, so none waits for another); the
@@ -54,7 +59,7 @@ __device__ __forceinline__ void norme_ligne(const float* __restrict__ x, const f
 #pragma unroll
         for (uint32_t u = 0; u < NORME_PAR_FIL; ++u) {
             const uint32_t i = t + u * FILS_NORME;
-            if (i < n) y[i] = float(double(xv[u]) * r * double(wv[u]));
+            if (i < n) y[place(i)] = float(double(xv[u]) * r * double(wv[u]));
         }
         return;
     }
@@ -64,6 +69,6 @@ __device__ __forceinline__ void norme_ligne(const float* __restrict__ x, const f
         s = fma(v, v, s);
     }
     const double r = 1.0 / sqrt(somme_arbre_f64(part, total, s) / double(n) + double(eps));
-    for (uint32_t i = t; i < n; i += FILS_NORME) y[i] = float(double(x[i]) * r * double(w[i]));
+    for (uint32_t i = t; i < n; i += FILS_NORME) y[place(i)] = float(double(x[i]) * r * double(w[i]));
 }
 }  // namespace trc

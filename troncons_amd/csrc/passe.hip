@@ -24,6 +24,16 @@ namespace trc {
 constexpr uint32_t Q8_OCTETS_BLOC = 34;  // f16 d, then 32 x i8 (ggml Q8_0)
 constexpr uint32_t FILS_PASSE = 256;
 static_assert(FILS_PASSE == FILS_NORME, "rmsnorm and the Q/K/V launch run the norm with its block size");
+// x of a Q8_0 product in LDS: a block's 8 float4 and one of padding, so that the lanes of a half, which read
+// one block each, spread over the banks (at 128 bytes a block every lane's reads meet in half of them).
+constexpr uint32_t Q8_X_PAS = 9;
+constexpr uint32_t Q8_X_COLONNES = 8192;      // columns of x that gemv_q8_0 stages (36 KiB)
+template <uint32_t X_PAS>
+struct PlaceQ8 {  // of x_i, in floats
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return i + 4u * (X_PAS - 8u) * (i >> 5); }
+};
+__host__ __device__ constexpr uint32_t octets_x_q8(uint32_t colonnes) { return 16u * Q8_X_PAS * (colonnes / 32u); }
+constexpr uint32_t Q8_X_LDS_MAX = 65536;      // bytes of x that a short product stages padded
 constexpr uint32_t FILS_ARGMAX = 1024;
 constexpr uint32_t ATTENTION_DIM = 64;
 constexpr uint32_t ATTENTION_POSITIONS_MAX = TRC_ATTENTION_POSITIONS_MAX;
@@ -90,7 +100,7 @@ __device__ inline double inv_freq_yarn(const trc_params_rope& p, uint32_t i, dou
 // 64-bit shift. The half-wavefront's rows are r0 .. r0 + LIGNES - 1; lane 0 hands each row's sum
 // (bias not added) to `ecrire(r, s)`. x may be in LDS or global memory.
 namespace trc {
-template <uint32_t LIGNES, uint32_t DEPLI, class Ecrire>
+template <uint32_t LIGNES, uint32_t DEPLI, uint32_t X_PAS, class Ecrire>  // X_PAS: float4 per block of x
 __device__ __forceinline__ void gemv_q8_0_rangees(const uint8_t* __restrict__ W, const float* __restrict__ x,
                                                   uint32_t R, uint32_t C, uint32_t r0, Ecrire ecrire) {
     const uint32_t voie = threadIdx.x & 31u;
@@ -138,7 +148,7 @@ __device__ __forceinline__ void gemv_q8_0_rangees(const uint8_t* __restrict__ W,
             float xv[32];
 #pragma unroll
             for (uint32_t k = 0; k < 8; ++k) {
-                const f32x4 t = x4[b * 8u + k];
+                const f32x4 t = x4[b * X_PAS + k];
                 xv[4 * k] = t.x;
                 xv[4 * k + 1] = t.y;
                 xv[4 * k + 2] = t.z;
@@ -176,28 +186,34 @@ constexpr uint32_t lignes_bloc() {
     return FILS_PASSE / 32u * LIGNES;
 }
 
-// x (C floats, C a multiple of 32) copied into the block's LDS with 16-byte loads.
+// x (C floats, C a multiple of 32) copied into the block's LDS with 16-byte loads, Q8_X_PAS per block.
 __device__ __forceinline__ void x_vers_lds(const float* __restrict__ x, f32x4* xs, uint32_t C) {
     const gptr<f32x4> x4 = glob<f32x4>(x);
-    for (uint32_t j = threadIdx.x; j < C / 4u; j += FILS_PASSE) xs[j] = x4[j];
+    for (uint32_t j = threadIdx.x; j < C / 4u; j += FILS_PASSE) xs[(j >> 3) * Q8_X_PAS + (j & 7u)] = x4[j];
     __syncthreads();
 }
 
 }  // namespace trc
 
-// One launch of y = W x (+ b). gemv_q8_0: four rows per half-wavefront, x read from global memory
-// (large matrices: the output head streams its weights with many waves resident);
-// gemv_q8_0_court: one row per half-wavefront, x staged in LDS when it fits (C <= QKV_COLONNES_MAX)
+// One launch of y = W x (+ b). gemv_q8_0: four rows per half-wavefront (large matrices: the output head
+// streams its weights with many waves resident), x in LDS up to Q8_X_COLONNES: read from device memory, a
+// lane's eight float4 of x lie in a line of their own, and those reads took more of the vector memory path
+// than the weights of four rows (201088 x 2880: 136 us, 4.5 TB/s, before; 111 us, 5.5 TB/s, with x in LDS;
+// 113 and 119 us with blocks of 512 and 1024 threads; two rows per half, x from device memory: 171 us);
+// gemv_q8_0_court: one row per half-wavefront, x staged in LDS when it fits (Q8_X_LDS_MAX)
 // and four of a lane's blocks' loads in flight (small matrices, where a launch has few blocks and
 // each wave's chain of loads sets the time).
-extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
+template <bool X_LDS>
+__global__ void __launch_bounds__(trc::FILS_PASSE)
 gemv_q8_0(const uint8_t* __restrict__ W, const float* __restrict__ x, const float* __restrict__ biais,
           float* __restrict__ y, float* __restrict__ residu, uint32_t R, uint32_t C) {
     using namespace trc;
     // the same rows, blocks and operation order as gemv_q8_0_rangees, with each row's window
     // loaded right before its use (fewer registers, more waves resident to stream the matrix)
+    extern __shared__ f32x4 xs[];
     const uint32_t voie = threadIdx.x & 31u;
     const uint32_t r0 = (blockIdx.x * (FILS_PASSE / 32u) + (threadIdx.x >> 5)) * 4u;
+    if (X_LDS) x_vers_lds(x, xs, C);
     if (r0 >= R) return;
     const uint32_t B = C / 32u;
     const uint64_t octets_ligne = uint64_t(B) * Q8_OCTETS_BLOC;
@@ -211,7 +227,7 @@ gemv_q8_0(const uint8_t* __restrict__ W, const float* __restrict__ x, const floa
         float xv[32];
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            const f32x4 t = x4[b * 8u + k];
+            const f32x4 t = X_LDS ? xs[b * Q8_X_PAS + k] : f32x4(x4[b * 8u + k]);
             xv[4 * k] = t.x;
             xv[4 * k + 1] = t.y;
             xv[4 * k + 2] = t.z;
@@ -274,11 +290,11 @@ gemv_q8_0_court(const uint8_t* __restrict__ W, const float* __restrict__ x, cons
             y[r] = v;
     };
     const uint32_t r0 = blockIdx.x * lignes_bloc<1>() + (threadIdx.x >> 5);
-    if (C <= QKV_COLONNES_MAX) {
+    if (octets_x_q8(C) <= Q8_X_LDS_MAX) {
         x_vers_lds(x, xs, C);
-        gemv_q8_0_rangees<1, 4>(W, reinterpret_cast<const float*>(xs), R, C, r0, ecrire);
+        gemv_q8_0_rangees<1, 4, Q8_X_PAS>(W, reinterpret_cast<const float*>(xs), R, C, r0, ecrire);
     } else {
-        gemv_q8_0_rangees<1, 4>(W, x, R, C, r0, ecrire);
+        gemv_q8_0_rangees<1, 4, 8>(W, x, R, C, r0, ecrire);
     }
 }
 
@@ -331,7 +347,8 @@ table_rope(trc_params_rope p, uint32_t position, double* __restrict__ table) {
 //    arithmetic) into y, and for k also into the cache slot, rounded to f16 (ecrire_kv);
 //  - v: eight consecutive rows into y and, rounded to f16, into the cache slot.
 // The values are those of rmsnorm, three gemv_q8_0, rope_yarn and ecrire_kv.
-extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
+template <uint32_t X_PAS>
+__global__ void __launch_bounds__(trc::FILS_PASSE)
 qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps, uint32_t C, trc::Q8Projections m,
          uint16_t* __restrict__ cache_k, uint16_t* __restrict__ cache_v, const double* __restrict__ table,
          uint32_t case_kv) {
@@ -341,7 +358,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
     __shared__ double total;
     __shared__ float paires[8];
     float* hh = reinterpret_cast<float*>(hh4);
-    norme_ligne(x, norme, hh, C, eps, part, &total);
+    norme_ligne(x, norme, hh, C, eps, part, &total, PlaceQ8<X_PAS>{});
     __syncthreads();
     const uint32_t hw = threadIdx.x >> 5;  // half-wavefront 0..7
     const uint32_t nbq = m.lignes[0] / 8u, nbk = m.lignes[1] / 8u, dkv = m.lignes[1];
@@ -351,7 +368,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
         if (j == 1u) bloc -= nbq;
         const uint32_t h = bloc / 8u, b = bloc % 8u;
         const float* bj = m.biais[j];
-        gemv_q8_0_rangees<1, 4>(m.w[j], hh, m.lignes[j], C, h * 64u + 32u * (hw >> 2) + 4u * b + (hw & 3u),
+        gemv_q8_0_rangees<1, 4, X_PAS>(m.w[j], hh, m.lignes[j], C, h * 64u + 32u * (hw >> 2) + 4u * b + (hw & 3u),
                                 [&](uint32_t r, float s) { paires[hw] = bj != nullptr ? s + bj[r] : s; });
         __syncthreads();
         if (threadIdx.x < 4u) {
@@ -371,7 +388,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
         bloc -= nbq + nbk;
         const float* bv = m.biais[2];
         float* yv = m.y[2];
-        gemv_q8_0_rangees<1, 4>(m.w[2], hh, m.lignes[2], C, bloc * 8u + hw, [&](uint32_t r, float s) {
+        gemv_q8_0_rangees<1, 4, X_PAS>(m.w[2], hh, m.lignes[2], C, bloc * 8u + hw, [&](uint32_t r, float s) {
             const float v = bv != nullptr ? s + bv[r] : s;
             yv[r] = v;
             cache_v[uint64_t(case_kv) * dkv + r] = f32_vers_f16(v);
@@ -726,14 +743,20 @@ constexpr uint32_t GEMV_COURT_LIGNES = 32768;
 void lancer_gemv(const uint8_t* W, const float* x, const float* biais, float* y, float* residu, uint32_t R, uint32_t C,
                  hipStream_t f) {
     if (R < GEMV_COURT_LIGNES) {
-        const size_t lds = C <= trc::QKV_COLONNES_MAX ? 4u * size_t(C) : 0u;
+        const size_t lds = trc::octets_x_q8(C) <= trc::Q8_X_LDS_MAX ? trc::octets_x_q8(C) : 0u;
         constexpr uint32_t rb = trc::lignes_bloc<1>();
         hipLaunchKernelGGL(gemv_q8_0_court, dim3((R + rb - 1) / rb), dim3(trc::FILS_PASSE), lds, f, W, x, biais, y,
                            residu, R, C);
     } else {
-        constexpr uint32_t rb = trc::lignes_bloc<4>();
-        hipLaunchKernelGGL(gemv_q8_0, dim3((R + rb - 1) / rb), dim3(trc::FILS_PASSE), 0, f, W, x, biais, y, residu, R,
-                           C);
+        if (C <= trc::Q8_X_COLONNES) {
+            constexpr uint32_t rb = trc::lignes_bloc<4>();
+            hipLaunchKernelGGL((gemv_q8_0<true>), dim3((R + rb - 1) / rb), dim3(trc::FILS_PASSE),
+                               trc::octets_x_q8(C), f, W, x, biais, y, residu, R, C);
+        } else {
+            constexpr uint32_t rb = trc::lignes_bloc<4>();
+            hipLaunchKernelGGL((gemv_q8_0<false>), dim3((R + rb - 1) / rb), dim3(trc::FILS_PASSE), 0,
+                               f, W, x, biais, y, residu, R, C);
+        }
     }
 }
 }  // namespace
@@ -919,11 +942,18 @@ int lancer_qkv_q8_0(trc_vue x, trc_vue norme, float eps, uint32_t colonnes, cons
         m.lignes[j] = lignes[j];
         blocs += lignes[j] / 8;
     }
-    hipLaunchKernelGGL(qkv_q8_0, dim3(blocs), dim3(FILS_PASSE), 4u * colonnes, flux_de(flux),
-                       reinterpret_cast<const float*>(x.adresse), reinterpret_cast<const float*>(norme.adresse), eps,
-                       colonnes, m, reinterpret_cast<uint16_t*>(cache_k.adresse),
-                       reinterpret_cast<uint16_t*>(cache_v.adresse), reinterpret_cast<const double*>(table.adresse),
-                       case_kv);
+    const bool etale = octets_x_q8(colonnes) <= Q8_X_LDS_MAX;
+    auto lancer = [&](auto noyau) {
+        hipLaunchKernelGGL(noyau, dim3(blocs), dim3(FILS_PASSE), etale ? octets_x_q8(colonnes) : 4u * colonnes,
+                           flux_de(flux), reinterpret_cast<const float*>(x.adresse),
+                           reinterpret_cast<const float*>(norme.adresse), eps, colonnes, m,
+                           reinterpret_cast<uint16_t*>(cache_k.adresse), reinterpret_cast<uint16_t*>(cache_v.adresse),
+                           reinterpret_cast<const double*>(table.adresse), case_kv);
+    };
+    if (etale)
+        lancer(qkv_q8_0<Q8_X_PAS>);
+    else
+        lancer(qkv_q8_0<8>);
     return apres_lancement("qkv_q8_0");
 }
 
