@@ -1192,10 +1192,12 @@ def main():
     noyaux = chrono_passes(fusion, lambda s: jeton(plan[s], s), n_chrono)
     sel_c = sel_i[:n_chrono, :, :k].cpu().numpy()
     # the CODES launches: fusion_codes (each tile's DELTA decoded in the kernel) or, for other tile
-    # lengths, fusion_gemv after the DELTA pass
-    gu_ms, gu_n = noyaux.get("fusion_codes/gate_up", noyaux.get("fusion_gemv/gate_up", (0.0, 1)))
-    bas_ms, bas_n = noyaux.get("fusion_codes/down", noyaux.get("fusion_gemv/down", (0.0, 1)))
-    nom_codes = "fusion_codes" if "fusion_codes/gate_up" in noyaux else "fusion_gemv"
+    # lengths, fusion_gemv after the DELTA pass; tiles so long that they are decoded into slots first
+    # have one decoding launch for all matrices, fusion_longues_codes (counted under gate/up)
+    nom_codes = next((n for n in ("fusion_codes", "fusion_gemv") if n + "/gate_up" in noyaux), "fusion_longues_codes")
+    longues = nom_codes == "fusion_longues_codes"
+    gu_ms, gu_n = noyaux[nom_codes if longues else nom_codes + "/gate_up"]
+    bas_ms, bas_n = (0.0, gu_n) if longues else noyaux[nom_codes + "/down"]
     # algorithmic bytes of a launch: the CODES_CTX streams it decodes, plus, when it decodes each
     # tile's DELTA itself (fusion_codes), the DELTA and MEDIANES streams
     lus = [couches[l].octets_codes + (couches[l].octets_echelles if nom_codes == "fusion_codes" else 0)
@@ -1208,7 +1210,8 @@ def main():
     roofline = {
         "bound": "hbm",
         "kernel": ("fusion_codes_gu (gate/up launch) + fusion_codes_swiglu (down launch)" if nom_codes == "fusion_codes"
-                   else "fusion_gemv (gate/up launch + down launch)"),
+                   else "fusion_gemv (gate/up launch + down launch)" if nom_codes == "fusion_gemv"
+                   else "fusion_longues_codes (one launch, all matrices)"),
         "achieved": round(float(atteint), 1), "peak": PIC_HBM, "unit": "GB/s",
         "frac": round(float(atteint / PIC_HBM), 4), "traffic": trafic,
         "traffic_source": (f"{FICHIER_PMC.relative_to(RACINE)}: rocprofv3 --pmc FETCH_SIZE then WRITE_SIZE per "
