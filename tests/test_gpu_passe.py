@@ -303,6 +303,28 @@ def test_attention_chunk_edges(k, n, tetes, kv, anneau, dec_v):
         assert np.abs(hote(s, np.float32) - ref64).max() <= 1e-6 * np.abs(ref64).max(), typ
 
 
+@pytest.mark.parametrize("n", [1, 20, 64, 100, 1100])
+def test_attention_nan_key_reaches_the_output(k, n):
+    """A NaN in one key makes the outputs of its kv head's query heads NaN, as a softmax over all the
+    positions does, also where no other position shares its lanes; the other heads keep their values."""
+    print(f"attention NaN n {n}", flush=True)
+    tetes, kv = 8, 2
+    rng = np.random.default_rng(n)
+    p = ParamsAttention(tetes, kv, 64, 0, n, 0, 0.125, 0)
+    q = rng.standard_normal(tetes * 64).astype(np.float32)
+    ck = (rng.standard_normal(n * kv * 64) * 0.5).astype(np.float16)
+    cv = rng.standard_normal(n * kv * 64).astype(np.float16)
+    puits = rng.standard_normal(tetes).astype(np.float32)
+    ref64 = attention_f64(q, ck.view(np.uint16), cv.view(np.uint16), puits, p).reshape(tetes, 64)[4:]
+    ck.reshape(n, kv, 64)[n // 2, 0, 9] = np.nan
+    for appel, typ in ((k.attention, np.float16), (k.attention_kvf32, np.float32)):
+        s = zeros(4 * 64 * tetes)
+        appel(vue(dev(q)), vue(dev(ck.astype(typ))), vue(dev(cv.astype(typ))), vue(dev(puits)), vue(s), p)
+        got = hote(s, np.float32).reshape(tetes, 64)
+        assert np.isnan(got[:4]).all(), typ
+        assert np.abs(got[4:] - ref64).max() <= 1e-6 * np.abs(ref64).max(), typ
+
+
 def test_argmax_ties_nan_and_random(k):
     v = np.zeros(100_000, np.float32)
     v[0] = np.nan

@@ -597,7 +597,8 @@ __device__ __forceinline__ void attention_tete(const float* __restrict__ q, cons
             // exp(-inf - -inf) would be NaN: no term has weight yet, as in the reference, whose maximum
             // includes the sink before any exponential (passe.cuh:306-371).
             const float alpha = m == -INFINITY ? 0.0f : expf(m - m2);  // 0 for the first chunk (m = -inf)
-            const float e = m2 == -INFINITY || j >= U ? 0.0f : expf(s_j - m2);
+            // (a NaN score is not the maximum's business, but its weight is NaN and so is the head's output)
+            const float e = s_j == -INFINITY || j >= U ? 0.0f : expf(s_j - m2);
             z = fmaf(z, alpha, e);
             m = m2;
             poids[w][lane] = e;  // read back by this group only, in program order
