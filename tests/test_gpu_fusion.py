@@ -507,3 +507,15 @@ def test_long_tiles_layer_expert_and_gemv(fz, N, d, r):
     vus = [couche([dev(bytes(casse)) if e == e0 else p for e, p in enumerate(parts)], t) for t in tailles]
     assert (vus[0][0].view(np.uint32) == avant.view(np.uint32)).all()
     assert vus[0][1] == vus[1][1] and vus[0][1][1] == 6 and vus[0][1][0] == vus[0][1][2] == 0
+
+
+def test_long_tiles_gemv_over_its_own_input(fz):
+    """y in x's memory: one matrix of 256-macro-step tiles still multiplies the x that the call was given."""
+    dims = DimsExpert.de([1024] * 3, [1024] * 3)
+    ex = Expert(77, dims, N_delta=256, N_codes=256)
+    x = O.synth_normale_bf16(77, 1, 0, 1024, 1.0)
+    attendu, _ = _gemv(fz, ex.partie, ex.luts, 1, 1024, 1024, x, 256, 256)
+    xy, ctl, tr = dev(x), zeros(16), zeros(fusion.taille_travail_gemv(1024, 1024, 256))
+    fz.gemv_fusionnee(vue(dev(ex.partie)), 1, vue(dev(ex.luts)), 1024, 1024, vue(xy), vue(xy), vue(ctl), vue(tr), 256, 256)
+    assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
+    assert np.abs(hote(xy, np.float32) - attendu).max() <= 2 * TOL * np.abs(attendu).max()

@@ -1110,7 +1110,10 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
         return TRC_OK;
     }
     const Taches tv = par_valeur(&t, 1);
-    if (longues(lignes, colonnes, 1, n_delta, n_codes) &&
+    // (the fused form reads all of x before its last launch writes y, the slots' one multiplies into y as
+    // it reads x: y over x keeps the fused form)
+    const bool separes = y.adresse >= x.adresse + 4ull * colonnes || x.adresse >= y.adresse + 4ull * lignes;
+    if (separes && longues(lignes, colonnes, 1, n_delta, n_codes) &&
         travail.octets >= trc_taille_travail_gemv_fusionnee(lignes, colonnes, n_codes)) {
         const Longues p = par_longues(tv, dims_matrice(lignes, colonnes), 1, travail.adresse);
         const int r = lancer_longues(p, lignes, colonnes, 1, n_delta, n_codes, l, ctl, f);
