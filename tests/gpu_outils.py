@@ -74,6 +74,46 @@ class Expert:
         return p, attendu
 
 
+def abimer_flux(partie: bytes, sorte: int, j: int, mal: str) -> bytes:
+    """The part with stream (sorte, matrix j) damaged (3 = DELTA, 4 = CODES_CTX):
+    bit     a bit flipped in the middle of the last tile's words;
+    milieu  the same in an interior tile;
+    debut   the last tile's start one word later;
+    loin    an interior tile's start just below 2^31 words, where 2 * start, as an offset in the stream, ends
+            at -16 modulo 2^32: the first reads past it lie at the very end of the 32-bit range."""
+    p = np.frombuffer(partie, np.uint8).copy()
+    n = int.from_bytes(p[10:12].tobytes(), "little")
+    (d,) = [64 + 16 * i for i in range(n) if p[64 + 16 * i] == sorte and p[64 + 16 * i + 1] == j]
+    dec = int.from_bytes(p[d + 4:d + 8].tobytes(), "little")
+    T, W = (int.from_bytes(p[dec + o:dec + o + 4].tobytes(), "little") for o in (8, 12))
+    assert T >= 3
+    debuts = p[dec + 16:dec + 16 + 4 * T].view(np.uint32)
+    mots = 16 + 132 * T
+    if mal in ("bit", "milieu"):
+        a, b = (int(debuts[T - 1]), W) if mal == "bit" else (int(debuts[1]), int(debuts[2]))
+        p[dec + mots + (a + b) // 2 * 2] ^= 0x10
+    elif mal == "debut":
+        assert debuts[T - 1] + 1 <= W
+        debuts[T - 1] += 1
+    else:
+        debuts[1] = (2**32 - 16 - mots) // 2
+    return p.tobytes()
+
+
+def freqs_un_contexte(blocs, dims: DimsExpert):
+    """A matrix's tables with the CODES_CTX table of all its codes for each of the three contexts: the
+    codes then decode the same whatever the scales (damage to DELTA stays in the scales)."""
+    freqs = []
+    for j in range(3):
+        B = dims.colonnes[j] // 32
+        f = codeur.tables([blocs[j]], dims.lignes[j], B)
+        b = np.array(blocs[j], np.uint8).reshape(-1, 17)
+        b[:, 0] = 127  # every scale the row's median: one context holds every block
+        f[1:] = codeur.tables([b.reshape(-1)], dims.lignes[j], B)[2]
+        freqs.append(f)
+    return freqs
+
+
 # Doubled E2M1 magnitudes (codes 0-7; bit 3 is the sign): the reference's k table.
 K_E2M1X2 = np.array([0.0, 1.0, 2.0, 3.0, 4.0, 6.0, 8.0, 12.0])
 

@@ -8,6 +8,8 @@ g++ and checked on the CPU:
 - elargir_u64, the widening of two `readfirstlane` results (int) into a 64-bit address: a low word
   with bit 31 set must not spill into the high word (a plain int -> uint64 conversion would
   sign-extend it), and a high word with bit 31 set must survive.
+- lecture_dans and dernier_depart, the bounds of the ring and chain readers, against 64-bit arithmetic: offsets from a
+  damaged tile start lie anywhere in 32 bits, those just below 2^32 included.
 """
 from __future__ import annotations
 
@@ -66,6 +68,25 @@ int main() {
     if (trc::elargir_u64(-1, 0) != 0x00000000FFFFFFFFull) { std::printf("elargir -1\n"); ++echecs; }
     // what the helper guards against: the int itself widened sign-extends
     if ((uint64_t(int64_t(bas)) >> 32) != 0xFFFFFFFFull) { std::printf("temoin\n"); ++echecs; }
+    // reads of 2 and 8 bytes: around both ends of the stream and of the 32-bit range, the offsets that a
+    // reader computes from a tile start (2 * debut past the words' origin, 8 bytes per lane), random ones
+    for (uint32_t fin : {0u, 1u, 7u, 8u, 16u, 17u, 4096u, 4097u, 0x7FFFFFF8u, 0xFFFFFFF7u, 0xFFFFFFF8u, 0xFFFFFFFFu})
+        for (uint32_t n : {2u, 8u, 16u}) {
+            std::vector<uint32_t> o;
+            for (uint32_t d = 0; d < 40; ++d)
+                for (uint32_t base : {0u, fin, 0u - 1u}) {
+                    o.push_back(base + d);
+                    o.push_back(base - d);
+                }
+            for (uint32_t debut : {0x7FFFFFF0u, 0x7FFFFFFFu, 0x80000000u, 0xFFFFFFFFu})
+                for (uint32_t lane = 0; lane < 64; ++lane) o.push_back(((148u + 2u * debut) & ~15u) + 8u * lane);
+            for (int i = 0; i < 1000; ++i) o.push_back(uint32_t(g()));
+            for (uint32_t x : o)
+                if (trc::lecture_dans(x, n, fin) != (uint64_t(x) + n <= fin) ||
+                    (fin >= n && (x <= trc::dernier_depart(n, fin)) != (uint64_t(x) + n <= fin))) {
+                    if (echecs++ < 10) std::printf("lecture_dans(%u, %u, %u)\n", x, n, fin);
+                }
+        }
     std::printf("%d\n", echecs);
     return echecs == 0 ? 0 : 1;
 }

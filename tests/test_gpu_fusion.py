@@ -15,7 +15,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 import oracle_ffi as O  # noqa: E402
-from gpu_outils import Expert, dev, hote, mlp_f64, poids_f64, vue, zeros  # noqa: E402
+from gpu_outils import Expert, abimer_flux, dev, freqs_un_contexte, hote, mlp_f64, poids_f64, vue, zeros  # noqa: E402
 from troncons_amd import codeur, fusion  # noqa: E402
 from troncons_amd import noyaux as K  # noqa: E402
 from troncons_amd.noyaux import DimsExpert  # noqa: E402
@@ -519,3 +519,47 @@ def test_long_tiles_gemv_over_its_own_input(fz):
     fz.gemv_fusionnee(vue(dev(ex.partie)), 1, vue(dev(ex.luts)), 1024, 1024, vue(xy), vue(xy), vue(ctl), vue(tr), 256, 256)
     assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
     assert np.abs(hote(xy, np.float32) - attendu).max() <= 2 * TOL * np.abs(attendu).max()
+
+
+@pytest.mark.parametrize("mal", ["bit", "debut", "loin"])
+@pytest.mark.parametrize("sorte", [3, 4])
+def test_long_tiles_layer_damaged_stream(fz, mal, sorte):
+    """A layer step over 256-macro-step tiles whose selected expert has a damaged down stream: the control
+    words are the oracle's decode of that part (a tile start near 2^31, which the oracle refuses, is
+    counted), and the other experts' part of the residual is not touched by it."""
+    print(f"damaged long-tile layer {mal} kind {sorte}", flush=True)
+    d, r, E, N = 2080, 1024, 2, 256
+    dims = DimsExpert.de([r, r, d], [d, d, r])
+    blocs, biais = codeur.synth_expert(79, 0, 0, dims)
+    freqs = freqs_un_contexte(blocs, dims)
+    luts = O.luts_couche([[freqs[j][t] for t in range(4)] for j in range(3)])
+    partie = codeur.partie(blocs, biais, freqs, dims, N_delta=N, N_codes=N)[0]
+    abime = abimer_flux(partie, sorte, 2, mal)
+    routeur = dev(np.zeros((E, d), np.uint16))  # equal logits: both experts, half each
+    x, avant = O.synth_normale_bf16(79, 4, 0, d, 1.0), O.synth_normale_bf16(79, 5, 0, d, 1.0)
+
+    def couche(octets):
+        parts = [dev(o) for o in octets]
+        table = dev(np.array([p.data_ptr() for p in parts], np.uint64))
+        rep, ctl0, res, idx, w, ctl = zeros(fusion.taille_repertoire(E)), zeros(16), dev(avant), zeros(32), zeros(32), zeros(16)
+        fz.monter_couche(vue(table), E, dims, vue(rep), vue(ctl0))
+        tr = dev(np.full(fusion.taille_travail_couche(dims, E, 2, N), 0xFF, np.uint8))
+        fz.couche_moe(vue(rep), E, vue(dev(luts)), dims, vue(routeur), None, vue(dev(x)), 2, vue(res), vue(idx), vue(w),
+                      vue(ctl), vue(tr), N, N)
+        return hote(res, np.float32), list(hote(ctl, np.uint32))
+
+    assert couche([partie, partie])[1] == [0, 0, 0, 0]
+    res, ctl = couche([partie, abime])
+    if mal == "loin":
+        assert ctl[0] + ctl[2] > 0 and ctl[1] == 0
+        return
+    oracle, octl = O.decoder_expert(abime, luts, dims.lignes, dims.colonnes)
+    assert ctl == list(octl) and octl[0] + octl[2] > 0
+    # rows of down whose blocks are all undamaged: half of each of two equal experts, within the tolerance
+    dj = K.disposition(dims, 2)
+    nb, sain = d * (r // 32), O.decoder_expert(partie, luts, dims.lignes, dims.colonnes)[0]
+    ok = (oracle == sain)[dj.base:dj.base + dj.pas]
+    rangs = ok[:16 * nb].reshape(d, -1).all(1) & ok[dj.echelles:dj.echelles + nb].reshape(d, -1).all(1)
+    attendu = avant + mlp_f64(blocs, biais, x.astype(np.float64)[:, None])[:, 0]
+    assert 0 < rangs.sum() < d
+    assert np.abs(res - attendu)[rangs].max() <= TOL * np.abs(attendu).max()

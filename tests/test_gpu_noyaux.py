@@ -11,7 +11,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 import oracle_ffi as O  # noqa: E402
-from gpu_outils import DEV, Expert, dev, hote, vue, zeros  # noqa: E402
+from gpu_outils import DEV, Expert, abimer_flux, dev, freqs_un_contexte, hote, vue, zeros  # noqa: E402
 from troncons_amd import codeur  # noqa: E402
 from troncons_amd import noyaux as K  # noqa: E402
 from troncons_amd.noyaux import DescDecodage, DescGemv, DimsExpert, VueCarte  # noqa: E402
@@ -380,3 +380,38 @@ def test_decoder_long_delta_tiles(k, N, dims, entropie):
     assert list(ctl) == [0, 0, 0, 0]
     oracle, octl = O.decoder_expert(partie, luts, d.lignes, d.colonnes)
     assert list(octl) == [0, 0, 0, 0] and (oracle == empl).all()
+
+
+@pytest.mark.parametrize("N", [64, 256])
+@pytest.mark.parametrize("mal", ["bit", "debut", "milieu", "loin"])
+@pytest.mark.parametrize("sorte", [3, 4])
+def test_decoder_damaged_long_tiles(k, N, mal, sorte):
+    """Streams of long tiles with damaged words or tile starts. Damage to the last tile is decoded as the
+    oracle decodes it, so that slot bytes and control words are equal (past the stream's last word both
+    read zeros); a damaged interior tile reads on into the next one's words where the oracle stops, so its
+    own blocks are left out of the comparison and it must be counted. A tile start near 2^31 is read as
+    words past the stream, never outside the part."""
+    print(f"damaged long tiles N {N} {mal} kind {sorte}", flush=True)
+    dims = DimsExpert.de([1024, 1024, 2080], [2080, 2080, 1024])
+    blocs, biais = codeur.synth_expert(78, 0, N, dims)
+    freqs = freqs_un_contexte(blocs, dims)
+    luts = O.luts_couche([[freqs[j][t] for t in range(4)] for j in range(3)])
+    partie, _ = codeur.partie(blocs, biais, freqs, dims, N_delta=N, N_codes=N)
+    bon, ctl = _decoder(k, partie, luts, dims=dims)
+    oracle, _ = O.decoder_expert(partie, luts, dims.lignes, dims.colonnes)
+    assert list(ctl) == [0, 0, 0, 0] and (bon == oracle).all()
+    for j in (0, 2):
+        abime = abimer_flux(partie, sorte, j, mal)
+        empl, ctl = _decoder(k, abime, luts, dims=dims)
+        assert ctl[1] == 0 and ctl[3] == 0
+        if mal in ("bit", "debut"):
+            oracle, octl = O.decoder_expert(abime, luts, dims.lignes, dims.colonnes)
+            assert list(ctl) == list(octl) and octl[0] + octl[2] > 0
+            assert (empl == oracle).all()
+        else:
+            assert ctl[0] + ctl[2] > 0
+            d = K.disposition(dims, j)  # tile 1: blocks N * 128 .. 2 N * 128 - 1 of DELTA, a sixteenth of CODES_CTX
+            a = d.base + (d.echelles if sorte == 3 else 0)
+            meme = empl == bon
+            meme[a + 128 * N:a + 256 * N] = True
+            assert meme.all()

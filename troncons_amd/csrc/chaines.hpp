@@ -47,7 +47,7 @@ constexpr uint32_t CHAINE_OCTETS = 2u * CHAINE_MOTS + 8u * (CHAINE_FICHES + CHAI
 // translation starts there, so that batches of 64 never straddle the rings' ends.
 struct Chaine {
     const uint8_t* flux;
-    uint32_t g0, fin;            // byte offsets in the stream: origin of the words, end of the stream
+    uint32_t g0, dernier;        // byte offsets in the stream: origin of the words, its last 8 bytes
     uint32_t a_brut, a_fiches;   // LDS: raw ring, records
     uint32_t a_lut;              // LDS: 4096 8-byte entries
     uint32_t lane;
@@ -62,7 +62,7 @@ struct Chaine {
     __device__ __forceinline__ u32x2 lire(uint32_t mot) const {
         const uint32_t o = g0 + 2u * mot + 8u * lane;
         u32x2 d = {0u, 0u};
-        if (o + 8u <= fin) d = *glob<u32x2>(flux + o);
+        if (o <= dernier) d = *glob<u32x2>(flux + o);
         return d;
     }
 
@@ -73,7 +73,7 @@ struct Chaine {
         const uint32_t mot0 = uint32_t(reinterpret_cast<const uint8_t*>(h.mots) - f.p) + 2u * debut;
         flux = f.p;
         g0 = mot0 & ~15u;
-        fin = f.longueur;
+        dernier = dernier_depart(8u, f.longueur);  // (its header, checked, is 16 bytes long)
         a_brut = zone;
         a_fiches = zone + 2u * CHAINE_MOTS;
         a_lut = lut;
@@ -172,7 +172,7 @@ struct Chaine {
         uint32_t x = y;
         if (y < L) {
             const uint32_t o = g0 + 2u * __builtin_amdgcn_mbcnt_lo(vote, p_vote);
-            x = (y << 16) | (o + 2u <= fin ? uint32_t(*glob<uint16_t>(flux + o)) : 0u);
+            x = (y << 16) | (o <= dernier + 6u ? uint32_t(*glob<uint16_t>(flux + o)) : 0u);
         }
         hors_l += x != L ? 1u : 0u;
         const uint32_t mot0 = uint32_t(reinterpret_cast<const uint8_t*>(h.mots) - flux) + 2u * debut;

@@ -736,7 +736,7 @@ struct AnneauR {
 __device__ __forceinline__ u32x2 lire_morceau_r(const AnneauR& a, uint32_t c, uint32_t v) {
     const uint32_t o = a.g0 + c * OCTETS_MORCEAU + v * 8u;
     u32x2 d = {0u, 0u};
-    if (o + 8u <= a.fin) d = *glob<u32x2>(a.flux + o);
+    if (lecture_dans(o, 8u, a.fin)) d = *glob<u32x2>(a.flux + o);
     return d;
 }
 
