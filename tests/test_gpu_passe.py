@@ -58,7 +58,7 @@ def test_gemv_q8_0_bit_exact_against_oracle(k, r, c):
     assert (_q8(k, o, x, None, r, c).view(np.uint32) == O.gemv_q8_0(o, x, None, r, c).view(np.uint32)).all()
 
 
-@pytest.mark.parametrize("r,c", [(33, 14560), (33, 14592), (32767, 96), (32768, 96), (32773, 352), (32769, 8192),
+@pytest.mark.parametrize("r,c", [(33, 14560), (33, 14592), (33, 16384), (32767, 96), (32768, 96), (32773, 352), (32769, 8192),
                                  (32769, 8224)])
 def test_gemv_q8_0_at_the_limits_of_its_forms(k, r, c):
     """Row counts around 32768 (one or four rows per half-wavefront) that do not fill a block, and widths

@@ -28,16 +28,16 @@ static_assert(FILS_PASSE == FILS_NORME, "rmsnorm and the Q/K/V launch run the no
 // one block each, spread over the banks (at 128 bytes a block every lane's reads meet in half of them).
 constexpr uint32_t Q8_X_PAS = 9;
 constexpr uint32_t Q8_X_COLONNES = 8192;      // columns of x that gemv_q8_0 stages (36 KiB)
-template <uint32_t X_PAS>
 struct PlaceQ8 {  // of x_i, in floats
-    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return i + 4u * (X_PAS - 8u) * (i >> 5); }
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const { return i + 4u * (Q8_X_PAS - 8u) * (i >> 5); }
 };
-__host__ __device__ constexpr uint32_t octets_x_q8(uint32_t colonnes) { return 16u * Q8_X_PAS * (colonnes / 32u); }
-constexpr uint32_t Q8_X_LDS_MAX = 65536;      // bytes of x that a short product stages padded
+constexpr uint32_t octets_x_q8(uint32_t colonnes) { return 16u * Q8_X_PAS * (colonnes / 32u); }
+// columns of x that a short product and the Q/K/V launch stage: 72 KiB, two blocks to a CU as with the 64 KiB
+// of unpadded x (2880 x 16384: 33.1 us with x from device memory, 21.4 unpadded, 17.0 padded)
+constexpr uint32_t Q8_X_COLONNES_COURT = 16384;
 constexpr uint32_t FILS_ARGMAX = 1024;
 constexpr uint32_t ATTENTION_DIM = 64;
 constexpr uint32_t ATTENTION_POSITIONS_MAX = TRC_ATTENTION_POSITIONS_MAX;
-constexpr uint32_t QKV_COLONNES_MAX = 16384;  // the normed row lives in LDS (64 KiB)
 
 // The three projections of qkv_q8_0 (q, k, v in that order).
 struct Q8Projections {
@@ -200,7 +200,7 @@ __device__ __forceinline__ void x_vers_lds(const float* __restrict__ x, f32x4* x
 // lane's eight float4 of x lie in a line of their own, and those reads took more of the vector memory path
 // than the weights of four rows (201088 x 2880: 136 us, 4.5 TB/s, before; 111 us, 5.5 TB/s, with x in LDS;
 // 113 and 119 us with blocks of 512 and 1024 threads; two rows per half, x from device memory: 171 us);
-// gemv_q8_0_court: one row per half-wavefront, x staged in LDS when it fits (Q8_X_LDS_MAX)
+// gemv_q8_0_court: one row per half-wavefront, x staged in LDS up to Q8_X_COLONNES_COURT
 // and four of a lane's blocks' loads in flight (small matrices, where a launch has few blocks and
 // each wave's chain of loads sets the time).
 template <bool X_LDS>
@@ -290,7 +290,7 @@ gemv_q8_0_court(const uint8_t* __restrict__ W, const float* __restrict__ x, cons
             y[r] = v;
     };
     const uint32_t r0 = blockIdx.x * lignes_bloc<1>() + (threadIdx.x >> 5);
-    if (octets_x_q8(C) <= Q8_X_LDS_MAX) {
+    if (C <= Q8_X_COLONNES_COURT) {
         x_vers_lds(x, xs, C);
         gemv_q8_0_rangees<1, 4, Q8_X_PAS>(W, reinterpret_cast<const float*>(xs), R, C, r0, ecrire);
     } else {
@@ -347,8 +347,7 @@ table_rope(trc_params_rope p, uint32_t position, double* __restrict__ table) {
 //    arithmetic) into y, and for k also into the cache slot, rounded to f16 (ecrire_kv);
 //  - v: eight consecutive rows into y and, rounded to f16, into the cache slot.
 // The values are those of rmsnorm, three gemv_q8_0, rope_yarn and ecrire_kv.
-template <uint32_t X_PAS>
-__global__ void __launch_bounds__(trc::FILS_PASSE)
+extern "C" __global__ void __launch_bounds__(trc::FILS_PASSE)
 qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps, uint32_t C, trc::Q8Projections m,
          uint16_t* __restrict__ cache_k, uint16_t* __restrict__ cache_v, const double* __restrict__ table,
          uint32_t case_kv) {
@@ -358,7 +357,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
     __shared__ double total;
     __shared__ float paires[8];
     float* hh = reinterpret_cast<float*>(hh4);
-    norme_ligne(x, norme, hh, C, eps, part, &total, PlaceQ8<X_PAS>{});
+    norme_ligne(x, norme, hh, C, eps, part, &total, PlaceQ8{});
     __syncthreads();
     const uint32_t hw = threadIdx.x >> 5;  // half-wavefront 0..7
     const uint32_t nbq = m.lignes[0] / 8u, nbk = m.lignes[1] / 8u, dkv = m.lignes[1];
@@ -368,7 +367,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
         if (j == 1u) bloc -= nbq;
         const uint32_t h = bloc / 8u, b = bloc % 8u;
         const float* bj = m.biais[j];
-        gemv_q8_0_rangees<1, 4, X_PAS>(m.w[j], hh, m.lignes[j], C, h * 64u + 32u * (hw >> 2) + 4u * b + (hw & 3u),
+        gemv_q8_0_rangees<1, 4, Q8_X_PAS>(m.w[j], hh, m.lignes[j], C, h * 64u + 32u * (hw >> 2) + 4u * b + (hw & 3u),
                                 [&](uint32_t r, float s) { paires[hw] = bj != nullptr ? s + bj[r] : s; });
         __syncthreads();
         if (threadIdx.x < 4u) {
@@ -388,7 +387,7 @@ qkv_q8_0(const float* __restrict__ x, const float* __restrict__ norme, float eps
         bloc -= nbq + nbk;
         const float* bv = m.biais[2];
         float* yv = m.y[2];
-        gemv_q8_0_rangees<1, 4, X_PAS>(m.w[2], hh, m.lignes[2], C, bloc * 8u + hw, [&](uint32_t r, float s) {
+        gemv_q8_0_rangees<1, 4, Q8_X_PAS>(m.w[2], hh, m.lignes[2], C, bloc * 8u + hw, [&](uint32_t r, float s) {
             const float v = bv != nullptr ? s + bv[r] : s;
             yv[r] = v;
             cache_v[uint64_t(case_kv) * dkv + r] = f32_vers_f16(v);
@@ -744,7 +743,7 @@ constexpr uint32_t GEMV_COURT_LIGNES = 32768;
 void lancer_gemv(const uint8_t* W, const float* x, const float* biais, float* y, float* residu, uint32_t R, uint32_t C,
                  hipStream_t f) {
     if (R < GEMV_COURT_LIGNES) {
-        const size_t lds = trc::octets_x_q8(C) <= trc::Q8_X_LDS_MAX ? trc::octets_x_q8(C) : 0u;
+        const size_t lds = C <= trc::Q8_X_COLONNES_COURT ? trc::octets_x_q8(C) : 0u;
         constexpr uint32_t rb = trc::lignes_bloc<1>();
         hipLaunchKernelGGL(gemv_q8_0_court, dim3((R + rb - 1) / rb), dim3(trc::FILS_PASSE), lds, f, W, x, biais, y,
                            residu, R, C);
@@ -921,7 +920,7 @@ namespace trc {
 int lancer_qkv_q8_0(trc_vue x, trc_vue norme, float eps, uint32_t colonnes, const trc_vue w[3],
                     const trc_vue biais[3], const trc_vue y[3], const uint32_t lignes[3], trc_vue cache_k,
                     trc_vue cache_v, trc_vue table, uint32_t case_kv, void* flux) {
-    TRC_VERIFIER(colonnes > 0 && colonnes % 32 == 0 && colonnes <= QKV_COLONNES_MAX, "qkv : %u colonnes", colonnes);
+    TRC_VERIFIER(colonnes > 0 && colonnes % 32 == 0 && colonnes <= Q8_X_COLONNES_COURT, "qkv : %u colonnes", colonnes);
     TRC_VERIFIER(x.adresse && norme.adresse && x.octets >= 4ull * colonnes && norme.octets >= 4ull * colonnes,
                  "qkv : x ou norme trop court");
     TRC_VERIFIER(table.adresse && table.adresse % 8 == 0 && table.octets >= 16 * 32, "qkv : table de rotation");
@@ -943,18 +942,11 @@ int lancer_qkv_q8_0(trc_vue x, trc_vue norme, float eps, uint32_t colonnes, cons
         m.lignes[j] = lignes[j];
         blocs += lignes[j] / 8;
     }
-    const bool etale = octets_x_q8(colonnes) <= Q8_X_LDS_MAX;
-    auto lancer = [&](auto noyau) {
-        hipLaunchKernelGGL(noyau, dim3(blocs), dim3(FILS_PASSE), etale ? octets_x_q8(colonnes) : 4u * colonnes,
-                           flux_de(flux), reinterpret_cast<const float*>(x.adresse),
-                           reinterpret_cast<const float*>(norme.adresse), eps, colonnes, m,
-                           reinterpret_cast<uint16_t*>(cache_k.adresse), reinterpret_cast<uint16_t*>(cache_v.adresse),
-                           reinterpret_cast<const double*>(table.adresse), case_kv);
-    };
-    if (etale)
-        lancer(qkv_q8_0<Q8_X_PAS>);
-    else
-        lancer(qkv_q8_0<8>);
+    hipLaunchKernelGGL(qkv_q8_0, dim3(blocs), dim3(FILS_PASSE), octets_x_q8(colonnes), flux_de(flux),
+                       reinterpret_cast<const float*>(x.adresse), reinterpret_cast<const float*>(norme.adresse), eps,
+                       colonnes, m, reinterpret_cast<uint16_t*>(cache_k.adresse),
+                       reinterpret_cast<uint16_t*>(cache_v.adresse), reinterpret_cast<const double*>(table.adresse),
+                       case_kv);
     return apres_lancement("qkv_q8_0");
 }
 
