@@ -335,13 +335,15 @@ def _al(n):
     return (n + 255) // 256 * 256
 
 
-@pytest.mark.parametrize("N", [(1, 16), (2, 16), (2, 32), ((2, 2, 1), (32, 32, 16)), (256, 256)])
+@pytest.mark.parametrize("N", [(1, 16), (2, 16), (2, 32), ((2, 2, 1), (32, 32, 16)), (256, 256), (16, 64),
+                               (63, 16), (64, 16)])
 def test_prefill_slots_bit_exact(fz, N):
     """The slot decoders' output itself, byte for byte: after a prefill whose routing chooses every
     expert, each expert's slot in the workspace holds exactly the code bytes and E8M0 scales of the
     oracle's canonical SoA slot (the reference decoder's output, -0 folded into +0). Tiles whose
     DELTA the CODES pass decodes (16/1, 16/2, 32/2, the bench's per-matrix encoding: the decode
-    step's tile machinery) and the reference encoder's 256/256 (the generic slot decoders). The
+    step's tile machinery), the reference encoder's 256/256 and DELTA tiles on both sides of the 64
+    macro-steps from which a block holds half as many (the generic slot decoders). The
     slots follow the piece counters, the per-expert counts and starts and the pair list, each
     256-byte aligned; the bias area of a slot is not written by the decoders and is not compared."""
     E, T, k = 4, 8, 4

@@ -34,7 +34,8 @@ constexpr int CTL_POINTEUR = 2;
 // Threads per block of the reference-API kernels (abi.rs:56-61 keeps these a launch detail).
 constexpr uint32_t FILS_ECHELLES = 256;  // 4 wavefronts: 4 long DELTA tiles, or 8 short ones
 constexpr uint32_t FILS_CODES = 256;     // 4 wavefronts = 8 CODES_CTX tiles
-// Tiles per block that the decoders' grids count on (kernels take any grid).
+// Tiles per block that the decoders' grids count on (kernels take any grid): these grids are made for the
+// reference encoder's tiles, without a look at the stream's tile length.
 constexpr uint32_t TUILES_BLOC_ECHELLES = 4;
 constexpr uint32_t TUILES_BLOC_CODES = 8;
 constexpr uint32_t FILS_BRUT = 256;

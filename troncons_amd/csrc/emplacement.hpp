@@ -77,6 +77,13 @@ struct LdsEchelles {
     __attribute__((aligned(16))) uint8_t med[MED_LDS_MAX];
 };
 
+// DELTA tiles per block of a launch over tiles of n_delta macro-steps: one per wavefront (chains) or two. A
+// grid of one per wavefront for short tiles too leaves half of the blocks with a LUT to expand and no
+// tile (8 gpt-oss experts, us with one / two per wavefront: tiles of 16 32.3 / 19.1, of 1 76 / 55).
+__host__ __device__ constexpr uint32_t tuiles_bloc_echelles(uint32_t fils, uint32_t n_delta) {
+    return n_delta >= CHAINE_N_MIN ? fils / 64u : fils / 32u;
+}
+
 // ----------------------------------------------------------------- DELTA -> E8M0 scales of the slot
 // e(block) = (med[row] + delta - 128) mod 256 (rans.rs:231-280); biases copied bit for bit.
 // The body, over located streams: fd (DELTA, header h), fm (MEDIANES), fb (BIAIS) of matrix j

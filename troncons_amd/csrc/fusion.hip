@@ -957,7 +957,8 @@ Longues par_longues(const Taches& t, const trc_dims_expert& dims, uint32_t exper
 int lancer_longues(const Longues& p, uint32_t R, uint32_t C, uint32_t jobs, uint32_t n_delta, uint32_t n_codes,
                    const uint32_t* l, uint32_t* ctl, hipStream_t f) {
     const uint64_t blocs = uint64_t(R) * (C / 32u);
-    TRC_LANCER(fusion_longues_echelles, dim3(grille_tuiles(blocs, n_delta, trc::TUILES_BLOC_ECHELLES), jobs),
+    const uint32_t tuiles_d = trc::tuiles_bloc_echelles(trc::FILS_ECHELLES, n_delta);
+    TRC_LANCER(fusion_longues_echelles, dim3(grille_tuiles(blocs, n_delta, tuiles_d), jobs),
                dim3(trc::FILS_ECHELLES), f, p, l, ctl);
     TRC_LANCER(fusion_longues_codes, dim3(grille_tuiles(16u * blocs, n_codes, trc::TUILES_BLOC_CODES), jobs),
                dim3(trc::FILS_CODES_SLOT), f, p, l, ctl);

@@ -1284,7 +1284,8 @@ extern "C" int trc_prefill_moe(trc_vue repertoire, uint32_t experts, trc_vue lut
             td = std::max<uint32_t>(td, uint32_t(((blocs + 127) / 128 + n_delta - 1) / n_delta));
             tc = std::max<uint32_t>(tc, uint32_t(((blocs * 16 + 127) / 128 + n_codes - 1) / n_codes));
         }
-        constexpr uint32_t tuiles_d = trc::TUILES_BLOC_ECHELLES, tuiles_c = trc::PF_FILS_CODES_SLOT / 32;
+        const uint32_t tuiles_d = trc::tuiles_bloc_echelles(trc::FILS_ECHELLES, n_delta);
+        constexpr uint32_t tuiles_c = trc::PF_FILS_CODES_SLOT / 32;
         TRC_LANCER(prefill_emplacements_echelles, dim3((td + tuiles_d - 1) / tuiles_d, 3, experts),
                    dim3(trc::FILS_ECHELLES), f, pp, l, ctl);
         TRC_LANCER(prefill_emplacements_codes, dim3((tc + tuiles_c - 1) / tuiles_c, 3, experts),
