@@ -287,9 +287,9 @@ def _couche_oracle(graine, E, k, x, avant, routeur):
     return oi, ow, ref, ref64
 
 
-@pytest.mark.parametrize("k", [1, 2, 6, 8])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 6, 8])
 def test_fused_moe_layer_topk_sizes_and_reused_workspace(fz, k):
-    """The bench's encoding (gate and up 2/32, down 1/16) at top-1, 2, 6 and 8. The workspace starts
+    """The bench's encoding (gate and up 2/32, down 1/16) at top-1, 2, 3, 5, 6 and 8. The workspace starts
     as 0xFF bytes and serves two steps in a row, the second adding into the first's residual with
     another x: nothing in the step may depend on the workspace's earlier contents."""
     E = 12
@@ -563,3 +563,38 @@ def test_long_tiles_layer_damaged_stream(fz, mal, sorte):
     attendu = avant + mlp_f64(blocs, biais, x.astype(np.float64)[:, None])[:, 0]
     assert 0 < rangs.sum() < d
     assert np.abs(res - attendu)[rangs].max() <= TOL * np.abs(attendu).max()
+
+
+@pytest.mark.parametrize("k,d,r", [(1, 1440, 1440), (3, 1440, 2016), (4, 1440, 1440), (5, 1440, 1440), (6, 1024, 1024)])
+@pytest.mark.parametrize("N", [(1, 16), (4, 8)])
+def test_launch_shapes_by_rounds(fz, N, k, d, r):
+    """Matrices whose CODES pass takes blocks of 256, 512 and 1024 threads, in one round of tile pairs and in
+    several, gate/up and down with the same or another size: the layer step and one expert against f64
+    from the uncompressed weights."""
+    print(f"launch shapes k {k} d {d} r {r} N {N}", flush=True)
+    E = 6
+    dims = DimsExpert.de([r, r, d], [d, d, r])
+    experts = [codeur.synth_expert(51, 0, e, dims) for e in range(E)]
+    freqs = [codeur.tables([x[0][j] for x in experts], dims.lignes[j], dims.colonnes[j] // 32) for j in range(3)]
+    luts = dev(O.luts_couche([[freqs[j][t] for t in range(4)] for j in range(3)]))
+    parts = [dev(codeur.partie(x[0], x[1], freqs, dims, expert=e, N_delta=N[0], N_codes=N[1])[0])
+             for e, x in enumerate(experts)]
+    table = dev(np.array([p.data_ptr() for p in parts], np.uint64))
+    routeur = np.stack([O.synth_normale_bf16(51, 3, e, d, 0.02) for e in range(E)])
+    r16, x = dev((routeur.view(np.uint32) >> 16).astype(np.uint16)), O.synth_normale_bf16(51, 4, 0, d, 1.0)
+    avant = O.synth_normale_bf16(51, 5, 0, d, 1.0)
+    oi, ow = O.routeur_topk(O.gemv_f32(routeur, x), k)
+    mlp = {int(e): mlp_f64(*experts[e], x.astype(np.float64)[:, None])[:, 0] for e in oi}
+    attendu = avant + sum(float(ow[i]) * mlp[int(e)] for i, e in enumerate(oi))
+    rep, ctl, res, idx, w = zeros(fusion.taille_repertoire(E)), zeros(16), dev(avant), zeros(32), zeros(32)
+    fz.monter_couche(vue(table), E, dims, vue(rep), vue(ctl))
+    tr = dev(np.full(fusion.taille_travail_couche(dims, E, k, N[1]), 0xFF, np.uint8))
+    fz.couche_moe(vue(rep), E, vue(luts), dims, vue(r16), None, vue(dev(x)), k, vue(res), vue(idx), vue(w), vue(ctl),
+                  vue(tr), *N)
+    assert (hote(idx, np.uint32)[:k] == oi).all() and list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
+    assert np.abs(hote(res, np.float32) - attendu).max() <= TOL * np.abs(attendu).max()
+    e0, s, ctl = int(oi[0]), zeros(4 * d), zeros(16)
+    tr = dev(np.full(fusion.taille_travail_expert(dims, N[1]), 0xFF, np.uint8))
+    fz.expert_fusionne(vue(parts[e0]), vue(luts), dims, vue(dev(x)), vue(s), vue(ctl), vue(tr), *N)
+    assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0]
+    assert np.abs(hote(s, np.float32) - mlp[e0]).max() <= TOL * np.abs(mlp[e0]).max()

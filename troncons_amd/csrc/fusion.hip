@@ -972,13 +972,16 @@ dim3 grille_gemv_long(uint32_t lignes, uint32_t jobs) {
 // Workspace piece of one matrix job in the internal-DELTA mode: its partial sums only.
 uint64_t pas_tache_interne(uint32_t R, uint32_t C) { return al(4ull * R * kmax_pour(C, 16)); }
 
-// Launch shape of a CODES pass over `jobs` matrices of R x C: 1024, 512 or 256 threads (32, 16 or 8
-// tiles) per block, the largest that still gives every CU of the chip a block, and at most about one
-// block per CU over all jobs (a block's LDS holds the three LUTs, so one fits a CU): wavefronts then
-// loop over further tile pairs instead of new blocks paying the LUT staging and the header reads.
-// "Every CU" up to a sixteenth: 254 blocks of 512 threads take gate and up of a gpt-oss expert at 16
-// macro-steps per tile in one round where 256 blocks of 256 threads need two (one expert: 51.8 -> 41.0 us).
-constexpr uint32_t CUS = 256, CUS_PRESQUE = CUS - CUS / 16u;
+// Launch shape of a CODES pass over `jobs` matrices of R x C: at most one block per CU over all jobs (a
+// block's LDS holds the three LUTs, so one fits a CU), whose wavefronts loop over further tile pairs
+// instead of new blocks paying the LUT staging and the header reads; and of 256, 512 or 1024 threads
+// (8, 16 or 32 tiles) the fewest that take no more rounds of pairs than more would: a round costs a tile's
+// chain of steps whether a SIMD runs one wavefront or four, and smaller blocks spread it over more CUs.
+// Measured with gate and up at 256 / 512 / 1024 threads, us per call (tiles 1/16), the rounds in brackets:
+// one expert 2880 x 2880 46.6 (2) / 39.4 (1) / 42.0 (1), 2880 x 1536 46.3 (2) / 37.9 (1) / 41.8 (1), 2048 x 2048
+// 37.0 (1) / 36.9 (1) / 40.2 (1); a top-4 layer 2880 x 2880 109 (8) / 65.5 (4) / 51.7 (2). (256 / jobs is rounded
+// down: a few blocks more than CUs are a second round of blocks, top-6 104 us with 264 blocks, 79.9 with 252.)
+constexpr uint32_t CUS = 256;
 
 struct FormeGemv {
     dim3 grille, bloc;
@@ -988,11 +991,15 @@ struct FormeGemv {
 FormeGemv forme_gemv(uint32_t R, uint32_t C, uint32_t N, uint32_t jobs) {
     const uint64_t octets = 16ull * R * (C / 32);
     const uint64_t T = ((octets + 127) / 128 + N - 1) / N;
-    uint32_t fils = trc::FILS_GEMV_MAX;
-    while (fils > 256 && ((T + fils / 32 - 1) / (fils / 32)) * jobs < CUS_PRESQUE) fils /= 2;
-    uint32_t gx = grille_tuiles(octets, N, fils / 32);
-    const uint32_t plafond = (CUS + jobs - 1) / jobs;
-    if (gx > plafond) gx = plafond;
+    const uint32_t plafond = std::max(CUS / jobs, 1u);
+    auto blocs = [&](uint32_t fils) { return std::min(grille_tuiles(octets, N, fils / 32), plafond); };
+    auto rondes = [&](uint32_t fils) {
+        const uint64_t paires = uint64_t(blocs(fils)) * (fils / 64);  // a round's
+        return ((T + 1) / 2 + paires - 1) / paires;
+    };
+    uint32_t fils = 256;
+    while (fils < trc::FILS_GEMV_MAX && rondes(fils) > rondes(trc::FILS_GEMV_MAX)) fils *= 2;
+    const uint32_t gx = blocs(fils);
     FormeGemv f;
     f.grille = dim3(gx, jobs);
     f.bloc = dim3(fils);
