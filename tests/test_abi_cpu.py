@@ -258,3 +258,21 @@ def test_streamed_layer_engine_refuses_bad_arguments_before_any_hip_call():
     assert h.value is None
     assert l.trc_diffusion_couche(None, 0, V(1 << 20, 4 * 2880), V(1 << 21, 4 * 2880), None, None) == 1
     assert l.trc_diffusion_jeton(None, V(1 << 20, 4 * 2880), V(1 << 21, 4 * 2880), None) == 1
+
+
+def test_fused_workspaces_of_long_tiles():
+    """From 128 macro-steps per tile the fused calls' queries cover the slots that the selected matrices are
+    decoded into: one matrix's for one product, an expert's, k experts' for a layer; rows of more than 3072
+    columns keep the fused form's size. The query for 127 covers the fused form of any longer tile."""
+    from troncons_amd import fusion
+
+    dims, large = DimsExpert.gpt_oss(), DimsExpert.de([256, 256, 3104], [3104, 3104, 256])
+    un = K.disposition_matrice(2880, 2880).pas
+    reste = 65536  # states and products of one matrix
+    for n in (128, 256, 65535):
+        assert un <= fusion.taille_travail_gemv(2880, 2880, n) <= un + reste
+        assert 3 * un <= fusion.taille_travail_expert(dims, n) <= 3 * (un + reste)
+        assert 12 * un <= fusion.taille_travail_couche(dims, 128, 4, n) <= 12 * (un + reste)
+        assert fusion.taille_travail_gemv(256, 3104, n) <= fusion.taille_travail_gemv(256, 3104, 127)
+        assert fusion.taille_travail_expert(large, n) <= fusion.taille_travail_expert(large, 127)
+        assert fusion.taille_travail_couche(large, 128, 4, n) <= fusion.taille_travail_couche(large, 128, 4, 127)

@@ -1066,16 +1066,20 @@ uint64_t travail_gemv_min(uint32_t lignes, uint32_t colonnes, uint32_t n_codes) 
     if (colonnes / 32 < 8 || n_codes == 0) return 0;
     return pas_tache(lignes, colonnes, n_codes);
 }
-// One matrix as the expert whose three matrices it is (only its own place is used).
-trc_dims_expert dims_matrice(uint32_t lignes, uint32_t colonnes) {
-    return trc_dims_expert{{lignes, lignes, lignes}, {colonnes, colonnes, colonnes}};
+// Matrix j as an expert whose other matrices are empty: a slot of one matrix. (The workspace query counts with
+// j = 0, which needs no less than the others.)
+trc_dims_expert dims_matrice(uint32_t j, uint32_t lignes, uint32_t colonnes) {
+    trc_dims_expert d{{0, 0, 0}, {0, 0, 0}};
+    d.lignes[j] = lignes;
+    d.colonnes[j] = colonnes;
+    return d;
 }
 }  // namespace
 
 extern "C" uint64_t trc_taille_travail_gemv_fusionnee(uint32_t lignes, uint32_t colonnes, uint32_t n_codes) {
     const uint64_t m = travail_gemv_min(lignes, colonnes, n_codes);
     if (m == 0 || !longues_possibles(n_codes, colonnes)) return m;
-    return std::max(m, octets_longues(dims_matrice(lignes, colonnes), 1, nullptr));
+    return std::max(m, octets_longues(dims_matrice(0, lignes, colonnes), 1, nullptr));
 }
 
 // Config 1: one matrix j of a part, y = W_j x + b_j, decoded in registers.
@@ -1123,7 +1127,7 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
     const bool separes = y.adresse >= x.adresse + 4ull * colonnes || x.adresse >= y.adresse + 4ull * lignes;
     if (separes && longues(lignes, colonnes, 1, n_delta, n_codes) &&
         travail.octets >= trc_taille_travail_gemv_fusionnee(lignes, colonnes, n_codes)) {
-        const Longues p = par_longues(tv, dims_matrice(lignes, colonnes), 1, travail.adresse);
+        const Longues p = par_longues(tv, dims_matrice(j, lignes, colonnes), 1, travail.adresse);
         const int r = lancer_longues(p, lignes, colonnes, 1, n_delta, n_codes, l, ctl, f);
         if (r != TRC_OK) return r;
         TRC_LANCER(fusion_longues_gemv<false>, grille_gemv_long(lignes, 1), dim3(trc::FILS_GEMV_LONG), f, p,
