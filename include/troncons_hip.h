@@ -255,11 +255,21 @@ int trc_combiner(trc_vue residu, trc_vue sorties, uint32_t pas, trc_vue poids, u
  * moteur/crates/trc-noyaux/noyaux/decodeur.cuh:227-231): the engine's caller of the expert hot
  * path is Modele::fin_couche (moteur/crates/trc-modele/src/lib.rs:533-553), which runs, per
  * selected expert, gemv(gate), gemv(up), swiglu_oai, gemv(down) over a decoded slot, then one
- * combiner. These entry points compute the same results from the coded part directly: the
- * decoded code bytes never reach device memory. `travail` is a caller-owned device workspace
- * (256-byte aligned) of at least the size the matching trc_taille_travail_* returns; n_delta and
- * n_codes are the macro-steps per tile of the DELTA and CODES_CTX streams (they size the grids
- * only: the kernels read the true N from every stream). Data errors go to `controle` as above. */
+ * combiner. These entry points compute the same results from the coded part directly. `travail` is a
+ * caller-owned device workspace (256-byte aligned) of the size the matching trc_taille_travail_*
+ * returns; n_delta and n_codes are the macro-steps per tile of the DELTA and CODES_CTX streams (the
+ * kernels read the true N from every stream: these size the grids and choose the form). Data errors go
+ * to `controle` as above.
+ *
+ * Two forms. Fused: the codes are decoded in registers where they are multiplied, and no decoded code
+ * byte reaches device memory. Slots, for long tiles (n_codes >= 128, rows of at most 3072 columns, and
+ * n_delta >= 64 or a launch of at most 2048 CODES_CTX tiles): the selected matrices are decoded into
+ * slots in `travail` and multiplied from there, about twice as fast at the reference encoder's 256/256.
+ * The queries return what both need. A smaller workspace is accepted as long as it holds the fused form,
+ * and the call then takes that form; the size that the query returns for n_codes = 127 always does, for
+ * the longer tiles too. Below 128 the query's size is the least accepted. (One product whose y overlaps
+ * its x takes the fused form too: only there is all of x read before y is written.) Each form gives the
+ * same bits on every call; the two add a row's products in different orders and agree to f32 rounding. */
 
 /* Workspace bytes of trc_gemv_fusionnee (0 if the shape is refused). */
 uint64_t trc_taille_travail_gemv_fusionnee(uint32_t lignes, uint32_t colonnes, uint32_t n_codes);
@@ -377,8 +387,10 @@ int trc_couche_moe_fusionnee(trc_vue repertoire, uint32_t experts, trc_vue luts,
 /* No counterpart in the reference. For callers that cannot allocate (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): trc_couche_moe_fusionnee with the library's
  * static device scratch (trc_octets_scratch() bytes, 16 MiB, one per device, held until the process
- * ends) as its workspace; it calls no allocating routine. A step needing more than the scratch
- * (trc_taille_travail_couche_moe) is a usage error. Every call on a device shares that device's
+ * ends) as its workspace; it calls no allocating routine. A step whose fused form needs more than the
+ * scratch is a usage error (trc_taille_travail_couche_moe for tiles below 128 macro-steps; for longer
+ * ones that query also covers the slots, and a step whose slots do not fit the scratch runs in the
+ * fused form). Every call on a device shares that device's
  * scratch: calls that overlap on one device (two streams, two threads) race; serialise them. The
  * scratch is taken on the device of `flux` (the current device if flux is null); its device address
  * is resolved once per device, by trc_contexte_creer (the library's set-up of a device) or else at

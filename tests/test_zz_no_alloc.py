@@ -107,6 +107,29 @@ def test_allocation_free_step_replays_from_a_graph():
     couche.c.liberer()
 
 
+@pytest.mark.parametrize("dims,k,fusionnee", [(DimsExpert.gpt_oss(), 4, True),
+                                              (DimsExpert.de([256, 256, 320], [320, 320, 256]), 2, False)])
+def test_allocation_free_step_of_long_tiles(dims, k, fusionnee):
+    """Tiles of 256 macro-steps: the slots of a top-4 gpt-oss layer do not fit the scratch, so the step takes the
+    fused form, with the bits of the allocating step on a workspace that holds no more than that form; a
+    small layer's slots fit, and the bits are those of the queried workspace."""
+    fz = fusion.Fusion()
+    E, N, graine = 6, (256, 256), 2053
+    assert (fusion.taille_travail_couche(dims, E, k, 256) > fusion.octets_scratch()) == fusionnee
+    couche = Couche(fz, graine, E, dims, N)
+    x = O.synth_normale_bf16(graine, 4, 0, dims.colonnes[0], 1.0)
+    residu0 = O.synth_normale_bf16(graine, 5, 0, dims.lignes[2], 0.5)
+    res, idx, w, ctl = dev(residu0), zeros(32), zeros(32), zeros(16)
+    tr = zeros(fusion.taille_travail_couche(dims, E, k, 127 if fusionnee else 256))
+    fz.couche_moe(vue(couche.rep), E, vue(couche.luts), dims, vue(couche.r16), None, vue(dev(x)), k, vue(res), vue(idx),
+                  vue(w), vue(ctl), vue(tr), *N)
+    b = _pas(fz, couche, E, dims, k, N, x, residu0, True)
+    assert list(hote(ctl, np.uint32)) == [0, 0, 0, 0] and list(b[3]) == [0, 0, 0, 0]
+    assert (hote(idx, np.uint32)[:k] == b[1]).all()
+    assert (hote(res, np.uint32) == b[0].view(np.uint32)).all() and np.abs(b[0] - residu0).max() > 0
+    couche.c.liberer()
+
+
 def test_step_larger_than_the_scratch_is_refused():
     fz = fusion.Fusion()
     dims, E, k, N = DimsExpert.gpt_oss(), 128, 8, (4, 16)

@@ -592,7 +592,7 @@ fusion_finir_combiner(trc::Taches taches) {
 }
 
 // ------------------------------------------------------------------------------------ long tiles
-// Streams of tiles of CHAINE_N_MIN macro-steps and more (the reference encoder writes 256): a matrix has
+// Streams of CODES_CTX tiles of LONGUES_N_MIN macro-steps and more (the reference encoder writes 256): a matrix has
 // too few tiles to fill the chip, and a launch that decodes some of the matrices takes as long as one
 // that decodes them all, the length of one tile's chain of dependent steps. So every selected matrix is
 // decoded at once into a slot of the workspace, DELTA then CODES_CTX (down's with gate's and up's,
@@ -975,8 +975,9 @@ uint64_t pas_tache_interne(uint32_t R, uint32_t C) { return al(4ull * R * kmax_p
 // Launch shape of a CODES pass over `jobs` matrices of R x C: at most one block per CU over all jobs (a
 // block's LDS holds the three LUTs, so one fits a CU), whose wavefronts loop over further tile pairs
 // instead of new blocks paying the LUT staging and the header reads; and of 256, 512 or 1024 threads
-// (8, 16 or 32 tiles) the fewest that take no more rounds of pairs than more would: a round costs a tile's
-// chain of steps whether a SIMD runs one wavefront or four, and smaller blocks spread it over more CUs.
+// (8, 16 or 32 tiles) the fewest that take no more rounds of pairs than more would: a round lasts a tile's
+// chain of steps, little longer with four wavefronts on a SIMD than with one, and smaller blocks spread over
+// more CUs.
 // Measured with gate and up at 256 / 512 / 1024 threads, us per call (tiles 1/16), the rounds in brackets:
 // one expert 2880 x 2880 46.6 (2) / 39.4 (1) / 42.0 (1), 2880 x 1536 46.3 (2) / 37.9 (1) / 41.8 (1), 2048 x 2048
 // 37.0 (1) / 36.9 (1) / 40.2 (1); a top-4 layer 2880 x 2880 109 (8) / 65.5 (4) / 51.7 (2). (256 / jobs is rounded

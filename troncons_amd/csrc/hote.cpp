@@ -55,8 +55,7 @@ static uint32_t tuiles(uint64_t octets) {
 
 static uint32_t au_moins_1(uint32_t v) { return v > 0 ? v : 1; }
 
-// abi.rs:137-141: one DELTA tile per 32-lane half-block unit of FILS_ECHELLES/32 tiles, one
-// CODES_CTX tile per FILS_CODES/32.
+// abi.rs:137-141: TUILES_BLOC_ECHELLES DELTA tiles per block, TUILES_BLOC_CODES CODES_CTX ones.
 extern "C" void trc_grilles_decodeur(const trc_dims_expert* dims, uint32_t g1[3], uint32_t g2[3]) {
     uint32_t td = 0, tc = 0;
     for (int j = 0; j < 3; ++j) {
