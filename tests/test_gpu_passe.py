@@ -276,10 +276,12 @@ def test_attention_first_chunk_of_minus_inf_scores(k):
     assert np.abs(got - ref).max() <= 3e-6 * np.abs(ref).max()
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 72, 127, 128, 129, 1023, 1024, 1025, 1100])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 72, 127, 128, 129, 255, 256, 257, 1023, 1024, 1025,
+                               1100])
 @pytest.mark.parametrize("tetes,kv,anneau,dec_v", [(64, 8, 0, 0), (6, 3, 0, 6), (4, 1, 5, 0), (8, 2, 70, 2)])
 def test_attention_chunk_edges(k, n, tetes, kv, anneau, dec_v):
-    """Position counts around the chunk sizes (8 up to 64 positions, then 64; 16 wavefronts a round),
+    """Position counts around the chunk sizes (8 up to 32 positions, then 64) and rounds (4 wavefronts up to
+    256 positions, then 16),
     heads that do not fill the XCDs, rings that wrap inside a chunk, values off 16-byte alignment, f16
     and f32 caches. Bound: a score is a 64-term f32 dot of unit-variance values and a weight's relative
     error is the score's absolute one (about 8 * 2^-24 * 64^0.5), averaged down over the positions:

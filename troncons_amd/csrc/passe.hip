@@ -444,12 +444,12 @@ ecrire_kv(const float* __restrict__ k, const float* __restrict__ v, uint16_t* __
 // exp(sink - M)), M the largest of the scores and the sink. Query head h reads kv head
 // h / (heads / kv heads).
 //
-// One block of 16 wavefronts per query head, one pass with a running softmax (Milakov & Gimelshein,
+// One block of 16 or 4 wavefronts per query head, one pass with a running softmax (Milakov & Gimelshein,
 // "Online normalizer calculation for softmax", 2018). A wavefront is eight groups of eight lanes;
 // a group takes one position at a time, lane j of it dimensions 8j .. 8j + 7 of its key and of its
 // value, so that a wavefront's load covers eight whole rows (a lane per row would touch 64 lines
 // for 16 bytes each). Chunks of 8 U positions go to the wavefronts in turn (chunk c to wavefront
-// c mod 16; position 8i + g of a chunk to group g). Each group keeps its own running maximum, sum
+// c mod VAGUES; position 8i + g of a chunk to group g). Each group keeps its own running maximum, sum
 // and outputs, rescaled by exp(old max - new max) once per chunk; lane i of a group takes the
 // exponential of its position 8i + g, the U weights reach its lanes through the wavefront's 64 LDS
 // words. Groups are merged by butterflies at the end, then the wavefronts and the sink in wavefront
@@ -458,14 +458,12 @@ ecrire_kv(const float* __restrict__ k, const float* __restrict__ v, uint16_t* __
 // What bounds it: a block reads its head's keys and values through one CU's vector memory path (2 MB
 // at 8192 positions) and spends about 250 VALU instructions per 64 positions on them; the blocks of a
 // kv head sit on one XCD, whose L2 then holds that head's rows for all of them. 64 heads over 8 kv
-// heads in f16: 274 -> 24 us at 8192 positions (one lane per position and four wavefronts before),
-// 9.2 -> 4.0 us at 128. The caches hold f16 (attention) or f32 (attention_kvf32).
+// heads in f16, us a launch (one lane per position and four wavefronts before): 274 -> 26.4 at 8192
+// positions, 8.6 -> 3.2 at 128, 3.4 -> 2.8 at 1. The caches hold f16 (attention) or f32 (attention_kvf32).
 namespace trc {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
-constexpr uint32_t FILS_ATTENTION = 1024;
-constexpr uint32_t VAGUES_ATTENTION = FILS_ATTENTION / 64u;
-constexpr uint32_t ATTENTION_COURTE = 64;  // positions up to which chunks hold 8 of them
+constexpr uint32_t VAGUES_ATTENTION = 16, VAGUES_ATTENTION_PEU = 4;
 
 // Dimensions 8j .. 8j + 7 of a stored row. LARGE: the row is 16-byte aligned.
 template <typename T>
@@ -521,7 +519,7 @@ __device__ __forceinline__ float somme_transposee(const float (&s)[8], uint32_t 
 }
 __device__ __forceinline__ float somme_transposee(const float (&s)[1], uint32_t) { return somme_groupe(s[0]); }
 
-template <typename T, uint32_t U, bool LARGE>
+template <typename T, uint32_t U, bool LARGE, uint32_t VAGUES>
 __device__ __forceinline__ void attention_tete(const float* __restrict__ q, const T* __restrict__ cache_k,
                                                const T* __restrict__ cache_v, const float* __restrict__ puits,
                                                float* __restrict__ sortie, const trc_params_attention& p) {
@@ -530,9 +528,9 @@ __device__ __forceinline__ void attention_tete(const float* __restrict__ q, cons
     // rows of a lane in flight: f16 a whole chunk's keys and values, f32 (twice the registers) half of
     // the keys, then half of the values
     constexpr uint32_t LOT = sizeof(T) == 2 || U < 4u ? U : U / 2u;
-    __shared__ float poids[VAGUES_ATTENTION][64];
-    __shared__ float sorties[VAGUES_ATTENTION][ATTENTION_DIM];
-    __shared__ float maxima[VAGUES_ATTENTION], sommes[VAGUES_ATTENTION];
+    __shared__ float poids[VAGUES][64];
+    __shared__ float sorties[VAGUES][ATTENTION_DIM];
+    __shared__ float maxima[VAGUES], sommes[VAGUES];
     const uint32_t t = threadIdx.x, w = uint32_t(__builtin_amdgcn_readfirstlane(int(t >> 6)));
     const uint32_t lane = t & 63u, g = lane >> 3, j = lane & 7u;
     // blocks go round the XCDs in turn: the query heads of one kv head to the same one (8 kv heads)
@@ -547,7 +545,7 @@ __device__ __forceinline__ void attention_tete(const float* __restrict__ q, cons
     const float puits_h = puits[h];
     if (RANGEES * w < n) {
         const f32x8 qv = lire_brut<true>(q + uint64_t(h) * ATTENTION_DIM + 8u * j);
-        for (uint32_t c0 = RANGEES * w; c0 < n; c0 += RANGEES * VAGUES_ATTENTION) {
+        for (uint32_t c0 = RANGEES * w; c0 < n; c0 += RANGEES * VAGUES) {
             const uint32_t c = case0 + c0, tour = p.anneau && c >= p.anneau ? p.anneau : 0u;  // wave-uniform
             const bool regulier = c0 + RANGEES <= n && (p.anneau == 0u || c - tour + RANGEES <= p.anneau);
             // the rows of positions c0 + 8i + g, i = i0 .. i0 + LOT - 1 (past the end: the last one's)
@@ -649,10 +647,10 @@ __device__ __forceinline__ void attention_tete(const float* __restrict__ q, cons
     if (t < ATTENTION_DIM) {
         float mg = puits_h;
 #pragma unroll
-        for (uint32_t v = 0; v < VAGUES_ATTENTION; ++v) mg = fmaxf(mg, maxima[v]);
+        for (uint32_t v = 0; v < VAGUES; ++v) mg = fmaxf(mg, maxima[v]);
         float zg = expf(puits_h - mg), og = 0.0f;
 #pragma unroll
-        for (uint32_t v = 0; v < VAGUES_ATTENTION; ++v) {
+        for (uint32_t v = 0; v < VAGUES; ++v) {
             const float fv = expf(maxima[v] - mg);
             zg = fmaf(sommes[v], fv, zg);
             og = fmaf(sorties[v][t], fv, og);
@@ -661,11 +659,11 @@ __device__ __forceinline__ void attention_tete(const float* __restrict__ q, cons
     }
 }
 
-template <typename T, uint32_t U, bool LARGE>
-__global__ void __launch_bounds__(FILS_ATTENTION)
+template <typename T, uint32_t U, bool LARGE, uint32_t VAGUES>
+__global__ void __launch_bounds__(64u * VAGUES)
 attention(const float* __restrict__ q, const T* __restrict__ cache_k, const T* __restrict__ cache_v,
           const float* __restrict__ puits, float* __restrict__ sortie, trc_params_attention p) {
-    attention_tete<T, U, LARGE>(q, cache_k, cache_v, puits, sortie, p);
+    attention_tete<T, U, LARGE, VAGUES>(q, cache_k, cache_v, puits, sortie, p);
 }
 }  // namespace trc
 
@@ -856,26 +854,38 @@ int verifier_attention(trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puit
 }  // namespace
 
 namespace {
-// One block per query head; chunks of 64 positions, or of 8 up to ATTENTION_COURTE positions, where
-// one 64-position chunk would leave 15 wavefronts idle (measured, us with chunks of 64 / of 8: 4.2 /
-// 4.0 at 64 positions, 4.0 / 4.5 at 128, 4.0 / 4.9 at 256, 4.4 / 6.1 at 512). Values that are not
-// 16-byte aligned (the contract asks it of the keys only) are read one by one.
+// One block per query head: 16 wavefronts in chunks of 64 positions; 4 as long as those have at most a
+// chunk each, as the wavefronts without one cost their start, their part of the merge and room on the CU;
+// and then chunks of 8 positions as long as the 4 have one each. Measured, us for 64 heads over 8 in f16 by
+// wavefronts/chunk: 16/8 3.9 at 1 position, 4.3 at 64, 4/8 2.8 at 1 and 2.9 at 32, 4/64 3.5 at 33, 3.1 at 64,
+// 3.2 at 128, 3.4 at 256, 16/64 4.0 at 65 and 128, 4.5 at 257. Values that are not 16-byte aligned (the
+// contract asks it of the keys only) are read one by one.
 template <typename T>
 int lancer_attention(const char* nom, trc_vue q, trc_vue cache_k, trc_vue cache_v, trc_vue puits, trc_vue sortie,
                      const trc_params_attention* p, void* flux) {
     const int r = verifier_attention(q, cache_k, cache_v, puits, sortie, p, sizeof(T));
     if (r != TRC_OK) return r;
-    auto lancer = [&](auto noyau) {
-        hipLaunchKernelGGL(noyau, dim3(p->tetes), dim3(trc::FILS_ATTENTION), 0, flux_de(flux),
+    auto lancer = [&](auto noyau, uint32_t vagues) {
+        hipLaunchKernelGGL(noyau, dim3(p->tetes), dim3(64u * vagues), 0, flux_de(flux),
                            reinterpret_cast<const float*>(q.adresse), reinterpret_cast<const T*>(cache_k.adresse),
                            reinterpret_cast<const T*>(cache_v.adresse), reinterpret_cast<const float*>(puits.adresse),
                            reinterpret_cast<float*>(sortie.adresse), *p);
     };
-    const bool long_ = p->fin - p->debut > trc::ATTENTION_COURTE, large = cache_v.adresse % 16 == 0;
-    if (large)
-        long_ ? lancer(trc::attention<T, 8, true>) : lancer(trc::attention<T, 1, true>);
+    const uint32_t n = p->fin - p->debut;
+    auto selon = [&](auto large) {
+        constexpr bool LARGE = decltype(large)::value;
+        constexpr uint32_t PEU = trc::VAGUES_ATTENTION_PEU, TOUTES = trc::VAGUES_ATTENTION;
+        if (n <= 8u * PEU)
+            lancer(trc::attention<T, 1, LARGE, PEU>, PEU);
+        else if (n <= 64u * PEU)
+            lancer(trc::attention<T, 8, LARGE, PEU>, PEU);
+        else
+            lancer(trc::attention<T, 8, LARGE, TOUTES>, TOUTES);
+    };
+    if (cache_v.adresse % 16 == 0)
+        selon(std::true_type{});
     else
-        long_ ? lancer(trc::attention<T, 8, false>) : lancer(trc::attention<T, 1, false>);
+        selon(std::false_type{});
     return trc::apres_lancement(nom);
 }
 }  // namespace
