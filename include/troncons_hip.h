@@ -263,7 +263,7 @@ int trc_combiner(trc_vue residu, trc_vue sorties, uint32_t pas, trc_vue poids, u
  *
  * Two forms. Fused: the codes are decoded in registers where they are multiplied, and no decoded code
  * byte reaches device memory. Slots, for long tiles (n_codes >= 128, rows of at most 3072 columns, and
- * n_delta >= 64 or a launch of at most 2048 CODES_CTX tiles): the selected matrices are decoded into
+ * unless the call has many tiles for n_delta to make up for): the selected matrices are decoded into
  * slots in `travail` and multiplied from there, about twice as fast at the reference encoder's 256/256.
  * The queries return what both need. A smaller workspace is accepted as long as it holds the fused form,
  * and the call then takes that form; the size that the query returns for n_codes = 127 always does, for

@@ -882,8 +882,8 @@ uint32_t kmax_pour(uint32_t colonnes, uint32_t n_codes) {
 
 uint64_t al(uint64_t x) { return (x + 255u) & ~uint64_t(255); }
 
-constexpr uint32_t LONGUES_N_MIN = 128;       // macro-steps per CODES_CTX tile from which tiles are long
-constexpr uint64_t LONGUES_TUILES = 8u * 256u;  // CODES_CTX tiles that one round of the decoding blocks takes
+constexpr uint32_t CUS = 256;
+constexpr uint32_t LONGUES_N_MIN = 128;  // macro-steps per CODES_CTX tile from which tiles are long
 
 uint32_t grille_tuiles(uint64_t octets, uint32_t N, uint32_t tuiles_par_bloc) {
     const uint64_t macro = (octets + 127) / 128;
@@ -921,18 +921,28 @@ uint64_t pas_tache(uint32_t R, uint32_t C, uint32_t n_codes) {
 bool delta_interne(uint32_t n_delta, uint32_t n_codes) { return trc::delta_dans_codes(n_delta, n_codes); }
 
 // Long tiles (fusion_longues_*): decoded into workspace slots. From 128 macro-steps per CODES_CTX tile (254
-// tiles in a 2880 x 2880 matrix) and rows that the GEMV stages in LDS; and where the launches' length is
-// a chain's: DELTA tiles that are decoded as chains, or all CODES_CTX tiles in one round of blocks.
-// Measured, us for a gpt-oss layer step, slots / fused, by k and delta/codes tiles: 4 256/256 262 / 608,
-// 8 256/256 408 / 613, 1 256/256 251 / 598, 4 128/128 232 / 342, 8 128/128 318 / 348, 4 16/128 201 / 211;
-// shorter tiles: 4 64/64 176 / 179, 4 16/64 166 / 126.
+// tiles in a 2880 x 2880 matrix), for rows that the GEMV stages in LDS, and by the rounds that the CODES_CTX
+// blocks take (one to a CU): each costs a tile's chain, 0.53 us a macro-step of N_codes. The fused form has two
+// such chains, gate and up's and then down's, and a DELTA pass longer by 0.8 us a macro-step of N_delta than
+// the chains are. So in one round slots, in two slots if the DELTA tiles are chains (else the forms are equal),
+// and from the third on if N_delta pays for the rounds past two: 0.53 / 0.8 of N_codes for each. Measured, us
+// for a 2880 x 2880 layer step, slots / fused, by k and delta/codes tiles: one round 2 16/128 116 / 198, 2 128/128
+// 147 / 329, 4 256/256 250 / 582; two 4 16/128 201 / 202 (here fused is taken), 4 64/128 205 / 256, 8 256/256
+// 386 / 585; three 8 64/128 290 / 263, 8 80/128 295 / 285, 8 88/128 298 / 295, 8 128/128 310 / 341, 8 96/192 369 / 342.
+// Shorter tiles: 4 64/64 176 / 179, 4 16/64 166 / 126.
 bool longues_possibles(uint32_t n_codes, uint32_t colonnes_max) {
     return n_codes >= LONGUES_N_MIN && colonnes_max <= trc::GEMV_X_COLONNES;
 }
-bool longues(uint32_t R, uint32_t C, uint32_t jobs, uint32_t n_delta, uint32_t n_codes) {
-    if (!longues_possibles(n_codes, C)) return false;
-    return n_delta >= trc::CHAINE_N_MIN ||
-           uint64_t(jobs) * grille_tuiles(16ull * R * (C / 32u), n_codes, 1) <= LONGUES_TUILES;
+// `blocs`: MXFP4 blocks of the largest of the `jobs` matrices.
+bool longues(uint64_t blocs, uint32_t colonnes_max, uint32_t jobs, uint32_t n_delta, uint32_t n_codes) {
+    if (!longues_possibles(n_codes, colonnes_max)) return false;
+    const uint64_t rondes = (uint64_t(jobs) * grille_tuiles(16u * blocs, n_codes, trc::TUILES_BLOC_CODES) + CUS - 1u) / CUS;
+    return rondes == 1u || (n_delta >= trc::CHAINE_N_MIN && 3u * uint64_t(n_delta) >= 2u * (rondes - 2u) * n_codes);
+}
+uint64_t blocs_max(const trc_dims_expert& d) {
+    uint64_t b = 0;
+    for (int j = 0; j < 3; ++j) b = std::max(b, uint64_t(d.lignes[j]) * (d.colonnes[j] / 32u));
+    return b;
 }
 // Workspace of `experts` experts' long tiles: states of their jobs, products, slots. rangs: rows per
 // product, a multiple of 64 floats.
@@ -953,10 +963,9 @@ Longues par_longues(const Taches& t, const trc_dims_expert& dims, uint32_t exper
     l.pas = trc_taille_emplacement(&dims);
     return l;
 }
-// Decoding launches of `jobs` matrices of at most R x C.
-int lancer_longues(const Longues& p, uint32_t R, uint32_t C, uint32_t jobs, uint32_t n_delta, uint32_t n_codes,
+// Decoding launches of `jobs` matrices of at most `blocs` blocks.
+int lancer_longues(const Longues& p, uint64_t blocs, uint32_t jobs, uint32_t n_delta, uint32_t n_codes,
                    const uint32_t* l, uint32_t* ctl, hipStream_t f) {
-    const uint64_t blocs = uint64_t(R) * (C / 32u);
     const uint32_t tuiles_d = trc::tuiles_bloc_echelles(trc::FILS_ECHELLES, n_delta);
     TRC_LANCER(fusion_longues_echelles, dim3(grille_tuiles(blocs, n_delta, tuiles_d), jobs),
                dim3(trc::FILS_ECHELLES), f, p, l, ctl);
@@ -982,8 +991,6 @@ uint64_t pas_tache_interne(uint32_t R, uint32_t C) { return al(4ull * R * kmax_p
 // one expert 2880 x 2880 46.6 (2) / 39.4 (1) / 42.0 (1), 2880 x 1536 46.3 (2) / 37.9 (1) / 41.8 (1), 2048 x 2048
 // 37.0 (1) / 36.9 (1) / 40.2 (1); a top-4 layer 2880 x 2880 109 (8) / 65.5 (4) / 51.7 (2). (256 / jobs is rounded
 // down: a few blocks more than CUs are a second round of blocks, top-6 104 us with 264 blocks, 79.9 with 252.)
-constexpr uint32_t CUS = 256;
-
 struct FormeGemv {
     dim3 grille, bloc;
     bool x_lds;
@@ -1126,10 +1133,10 @@ extern "C" int trc_gemv_fusionnee(trc_vue partie, uint32_t j, trc_vue luts, uint
     // (the fused form reads all of x before its last launch writes y, the slots' one multiplies into y as
     // it reads x: y over x keeps the fused form)
     const bool separes = y.adresse >= x.adresse + 4ull * colonnes || x.adresse >= y.adresse + 4ull * lignes;
-    if (separes && longues(lignes, colonnes, 1, n_delta, n_codes) &&
+    if (separes && longues(uint64_t(lignes) * B, colonnes, 1, n_delta, n_codes) &&
         travail.octets >= trc_taille_travail_gemv_fusionnee(lignes, colonnes, n_codes)) {
         const Longues p = par_longues(tv, dims_matrice(j, lignes, colonnes), 1, travail.adresse);
-        const int r = lancer_longues(p, lignes, colonnes, 1, n_delta, n_codes, l, ctl, f);
+        const int r = lancer_longues(p, uint64_t(lignes) * B, 1, n_delta, n_codes, l, ctl, f);
         if (r != TRC_OK) return r;
         TRC_LANCER(fusion_longues_gemv<false>, grille_gemv_long(lignes, 1), dim3(trc::FILS_GEMV_LONG), f, p,
                    reinterpret_cast<const float*>(x.adresse), reinterpret_cast<float*>(y.adresse));
@@ -1216,9 +1223,10 @@ extern "C" int trc_expert_fusionne(trc_vue partie, trc_vue luts, const trc_dims_
         return TRC_OK;
     }
     const Taches trois = par_valeur(t, 3), bas = par_valeur(t + 2, 1);
-    if (longues(Rm, Cm, 3, n_delta, n_codes) && travail.octets >= trc_taille_travail_expert_fusionne(dims, n_codes)) {
+    if (longues(blocs_max(*dims), Cm, 3, n_delta, n_codes) &&
+        travail.octets >= trc_taille_travail_expert_fusionne(dims, n_codes)) {
         const Longues p = par_longues(trois, *dims, 1, base);
-        r = lancer_longues(p, Rm, Cm, 3, n_delta, n_codes, l, ctl, f);
+        r = lancer_longues(p, blocs_max(*dims), 3, n_delta, n_codes, l, ctl, f);
         if (r != TRC_OK) return r;
         TRC_LANCER(fusion_longues_gemv<false>, grille_gemv_long(R, 2), dim3(trc::FILS_GEMV_LONG), f, p,
                    reinterpret_cast<const float*>(x.adresse), static_cast<float*>(nullptr));
@@ -1419,10 +1427,10 @@ int couche_moe(trc_vue repertoire, uint32_t experts, trc_vue luts, const trc_dim
         TRC_LANCER(fusion_finir_combiner, dim3((D + 255) / 256), dim3(256), f, t_bas);
         return TRC_OK;
     }
-    if (longues(Rm, std::max(C, R), 3 * k, n_delta, n_codes) &&
+    if (longues(blocs_max(*dims), std::max(C, R), 3 * k, n_delta, n_codes) &&
         travail.octets >= trc_taille_travail_couche_moe(dims, experts, k, n_codes)) {
         const Longues pl = par_longues(t_delta, *dims, k, morceaux);
-        r = lancer_longues(pl, Rm, std::max(C, R), 3 * k, n_delta, n_codes, l, ctl, f);
+        r = lancer_longues(pl, blocs_max(*dims), 3 * k, n_delta, n_codes, l, ctl, f);
         if (r != TRC_OK) return r;
         TRC_LANCER_N("fusion_longues_gemv/gate_up", fusion_longues_gemv<false>, grille_gemv_long(R, 2 * k),
                      dim3(trc::FILS_GEMV_LONG), f, pl, reinterpret_cast<const float*>(x.adresse),
