@@ -597,8 +597,8 @@ fusion_finir_combiner(trc::Taches taches) {
 // that decodes them all, the length of one tile's chain of dependent steps. So every selected matrix is
 // decoded at once into a slot of the workspace, DELTA then CODES_CTX (down's with gate's and up's,
 // where the fused form must decode down after the SwiGLU), and the products are GEMVs over the slots.
-// Measured for a top-4 gpt-oss layer at 256/256: 612 -> 262 us (DELTA pass 308, gate/up 143 and down 141 us one
-// after the other before; DELTA 105, CODES_CTX 135, the GEMVs 9 and 8 now).
+// Measured for a top-4 gpt-oss layer at 256/256: 612 -> 257 us (DELTA pass 308, gate/up 143 and down 141 us one
+// after the other before; DELTA 104, CODES_CTX 136, the GEMVs 9 and 8 now).
 struct Longues {
     trc::Taches taches;      // TACHES_MOE_DELTA (job y = expert y / 3, matrix y % 3) or local jobs
     uint64_t emplacements;   // slot of selected expert 0
